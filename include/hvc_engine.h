@@ -170,10 +170,12 @@ hvc_status hvc_batch_upload_synapses(hvc_ctx* ctx, int net, const hvc_synapses* 
 typedef struct {
     int integrate_block;   /* threads per block of the integration kernel: 64, 128, 256 */
     int i_lanes;           /* HVC-I DP8: 3 = eight lanes per neuron, 2 = four lanes, 1 = five lanes,
-                              0 = one thread per neuron */
+                              0 = one thread per neuron (FP64 form: 1 to 3 are all eight lanes) */
     int deliver_block;     /* 64, 128, 256 */
     int sync_block;        /* 64 .. 512 */
-    int ra_lanes;          /* HVC-RA RK4: 1 = four lanes per neuron, 0 = one thread per neuron */
+    int ra_lanes;          /* FP32 form, HVC-RA RK4: 1 = four lanes per neuron, 0 = one thread per neuron.
+                              FP64 form, both HVC-RA models: 1 = eight lanes per neuron, 0 = eight lanes for
+                              networks small enough to gain by it, else one thread */
     int deliver_lists;     /* 1 = the delivery visits only the neurons that spiked in the window or
                               still have spikes in flight (lists kept on the device), 0 = it reads
                               every neuron's queue state each window */

@@ -1,0 +1,71 @@
+"""The FP64 octet steppers (eight lanes per neuron) where they can go wrong, bit
+for bit against the oracle: partly filled waves, steps that leave the range of
+the fast quotients and repeat with IEEE division, and a network too large for
+octets, which takes one thread per neuron."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from oracle_lib import OracleSim
+
+pytestmark = pytest.mark.gpu
+
+
+def _compare(net, trial_ms, trials=1, tuning=None, **kw):
+    from unsupervised_growth_amd.engine import Engine
+    ora = OracleSim(net, trial_ms=trial_ms, **kw)
+    with Engine(trial_ms=trial_ms, **kw) as eng:
+        eng.upload(net)
+        if tuning:
+            eng.set_tuning(**tuning)
+        for k in range(trials):
+            tr = dict(mode=0, trial_index=k, first_trial=k == 0, mean_injection_time=5.0)
+            o, r = ora.run_trial(**tr), eng.run_trial(want_state=True, **tr)
+            for kind in ("soma", "dend", "interneuron"):
+                for a, b in zip(getattr(r, kind), o[kind]):
+                    np.testing.assert_array_equal(a, b)
+            np.testing.assert_array_equal(r.ra_state, o["ra_state"])
+            np.testing.assert_array_equal(r.i_state, o["i_state"])
+    return r
+
+
+@pytest.mark.parametrize("model", [0, 1])
+@pytest.mark.parametrize("n_ra,n_i", [(1, 1), (7, 9), (8, 8), (65, 17)])
+def test_partly_filled_waves(model, n_ra, n_i):
+    from unsupervised_growth_amd.network import random_network
+    net = random_network(n_ra, n_i, n_train=4, p_ra2i=0.5, p_i2ra=0.5, seed=n_ra)
+    _compare(net, 60.0, trials=2, ra_model=model, ra_poisson=model,
+             tuning=dict(integrate_block=64 if n_ra < 60 else 256))
+
+
+@pytest.mark.parametrize("model", [0, 1])
+def test_steps_out_of_the_fast_range(model):
+    """Resting potentials far out (gate arguments and voltages beyond the fast
+    range, overflowing exponentials) and conductances under which the HVC-I
+    stepper diverges through every magnitude to infinity and NaN."""
+    from unsupervised_growth_amd.network import random_network
+    net = random_network(24, 12, n_train=12, p_ra2i=0.6, p_i2ra=0.6, seed=2)
+    erest = net.erest.copy()
+    erest[:4] = [-3.0e4, 3.0e4, -1.0e9, 2.0e5]
+    net = dataclasses.replace(net, erest=erest, ra2i_w=net.ra2i_w * 1.0e5)
+    r = _compare(net, 30.0, ra_model=model)
+    assert r.bad_values == -1 and not np.isfinite(r.i_state).all() and (abs(r.ra_state[:4, 0]) > 2000).any()
+
+
+@pytest.mark.parametrize("model,n_ra", [(0, 32769), (1, 16385)])
+def test_large_network_takes_one_thread_per_neuron(model, n_ra):
+    from unsupervised_growth_amd.network import random_network
+    small = random_network(5, 3, n_train=2, p_ra2i=0.5, p_i2ra=0.5, seed=4, rr=2)
+    pad = n_ra - 5
+
+    def more(ptr):
+        return np.concatenate([ptr, np.full(pad, ptr[-1], np.int32)])
+
+    z = np.zeros(pad, np.int32)
+    net = dataclasses.replace(small, n_ra=n_ra, ra2i_ptr=more(small.ra2i_ptr), rr_ptr=more(small.rr_ptr),
+                              act_cnt=np.concatenate([small.act_cnt, z]), sup_cnt=np.concatenate([small.sup_cnt, z]),
+                              remodeled=np.concatenate([small.remodeled, z]),
+                              erest=np.concatenate([small.erest, np.linspace(-90.0, -60.0, pad)]),
+                              gca=np.concatenate([small.gca, np.linspace(0.0, 60.0, pad)]))
+    _compare(net, 3.0, ra_model=model)

@@ -1477,12 +1477,14 @@ extern "C" hvc_status hvc_autotune(hvc_ctx* ctx, int windows, hvc_tuning* best, 
     double ms[3], best_ms[3];
     hvc_status r;
     // integrate: block size and the HVC-I and HVC-RA layouts (four, five and
-    // eight lanes per HVC-I neuron exist for DP8 only, four per HVC-RA neuron
-    // for RK4 only)
+    // eight lanes per HVC-I neuron exist for DP8 only, FP32's four per HVC-RA
+    // neuron for RK4 only; in FP64 every layout with several lanes is eight)
     double bi = 1e30;
     Tuning ti = tu;
-    for (int ra_lanes = (ctx->prm.ra_model == 1 ? 1 : 0); ra_lanes >= 0; --ra_lanes)
+    const bool f64 = ctx->prm.precision == 0;
+    for (int ra_lanes = (ctx->prm.ra_model == 1 || f64 ? 1 : 0); ra_lanes >= 0; --ra_lanes)
         for (int lanes = (ctx->prm.i_model == 0 ? 3 : 0); lanes >= 0; --lanes) {
+            if (f64 && (lanes == 1 || lanes == 2)) continue;
             for (int bs : {64, 128, 256}) {
                 Tuning c = tu;
                 c.integrate_block = bs;

@@ -11,6 +11,7 @@
 
 #include "hvc_internal.h"
 #include "hvc_neuron.hip.h"
+#include "hvc_oct64.hip.h"
 #include "hvc_stdp.hip.h"
 
 namespace hvc {
@@ -79,9 +80,9 @@ __device__ __forceinline__ void ra_step_debraband(RAState& s, real el, real gca,
                      (ra_debraband<true>(bad, s, el, gca, u, J1s, J2s, J1d, J2d, E_dt, E_half)))
 }
 
-template <bool LANES = false>
+template <bool LANES = false, class Slot = int>
 __device__ __forceinline__ void ra_step_runge4(RAState& s, real el, real gca, const RAUniform& u, real E_third,
-                                               real E_twothird, real E_dt, const RAGateSlot* sl = nullptr)
+                                               real E_twothird, real E_dt, const Slot* sl = nullptr)
 {
     HVC_GUARDED_STEP(RAState, (ra_runge4<false, LANES>(bad, s, el, gca, u, sl, E_third, E_twothird, E_dt)),
                      (ra_runge4<true, LANES>(bad, s, el, gca, u, sl, E_third, E_twothird, E_dt)))
@@ -97,31 +98,29 @@ __device__ __forceinline__ void i_step(IState& s, real dt, const Row& row)
     }
 }
 
+#ifdef HVC_FP32
 template <class Row>
 __device__ __forceinline__ void i_step_lanes(IState& s, real& xlo, int role, int base, real dt, const Row& row)
 {
-    HVC_GUARDED_STEP(IState, (i_dp8_lanes<false>(bad, s, xlo, role, base, dt, row)),
-                     (i_dp8_lanes<true>(bad, s, xlo, role, base, dt, row)))
+    Guard bad;
+    i_dp8_lanes<false>(bad, s, xlo, role, base, dt, row);
 }
 
 template <class Row>
 __device__ __forceinline__ void i_step_quad(IState& s, real& xlo, real& wlo, int role, const GateSlot& ga,
                                             const GateSlot& gb, real dt, const Row& row)
 {
-    // the low parts are state too: a repeated step starts from their saved values
-    real xlo0 = xlo, wlo0 = wlo;
-    HVC_GUARDED_STEP(IState, (i_dp8_quad<false>(bad, s, xlo, wlo, role, ga, gb, dt, row)),
-                     (xlo = xlo0, wlo = wlo0, i_dp8_quad<true>(bad, s, xlo, wlo, role, ga, gb, dt, row)))
+    Guard bad;
+    i_dp8_quad<false>(bad, s, xlo, wlo, role, ga, gb, dt, row);
 }
 template <class Row>
 __device__ __forceinline__ void i_step_oct(IState& s, real& xo, real& xlo, int q, const GateSlot& g, real dt,
                                            const Row& row)
 {
-    // the lane's variable and its low part are state too
-    real xo0 = xo, xlo0 = xlo;
-    HVC_GUARDED_STEP(IState, (i_dp8_oct<false>(bad, s, xo, xlo, q, g, dt, row)),
-                     (xo = xo0, xlo = xlo0, i_dp8_oct<true>(bad, s, xo, xlo, q, g, dt, row)))
+    Guard bad;
+    i_dp8_oct<false>(bad, s, xo, xlo, q, g, dt, row);
 }
+#endif
 #undef HVC_GUARDED_STEP
 
 // state variables between HBM (FP64) and registers: the FP32 form keeps a
@@ -397,8 +396,77 @@ __device__ __forceinline__ void wl_enlist(const NetDev& nd, int role, bool spike
 constexpr int kRALanes = 4;                      // lanes per HVC-RA neuron (RK4 form)
 constexpr int kRANeuronsPerWave = 64 / kRALanes;  // 16 neurons
 
+// the postsynaptic events of an HVC-RA neuron as a window finds them
+struct RAPosts {
+    int growth, count;
+    double last;      // the latest one's time (count > 0)
+};
+// post events detected in the previous window become visible now (NGS:9385-9386);
+// lead: the lane that keeps neuron ii's events
+__device__ __forceinline__ RAPosts ra_posts_begin(const NetDev& nd, const Win& win, int growth, int ii, int t0,
+                                                  bool lead)
+{
+    RAPosts p{growth, nd.post_cnt[ii], 0.0};
+    if (growth && lead) {
+        int pend = nd.post_pend[ii];
+        if (pend > 0) {
+            double cs = win.clk(t0 - 1);
+            for (int q = 0; q < pend; ++q) {
+                nd.post_ring[(size_t)ii * kPostRing + (p.count % kPostRing)] = cs;
+                ++p.count;
+            }
+            if (pend > 2) atomicOr(nd.err, (unsigned)kErrPostRing);
+            nd.post_cnt[ii] = p.count;
+            nd.post_pend[ii] = 0;
+        }
+        if (p.count > 0) p.last = nd.post_ring[(size_t)ii * kPostRing + ((p.count - 1) % kPostRing)];
+    }
+    return p;
+}
+// after the steps: the spike logs, the delivery lists and the new postsynaptic
+// events (NGS:8956-8967; a window's events become visible in the next window,
+// so each spike is tested against the events of earlier windows only, as in
+// the step loop).  smask / dmask: the lane's somatic / dendritic spikes of
+// neuron i.  Returns the lane's new events.
+__device__ __forceinline__ int ra_window_logs(const NetDev& nd, const Win& win, const RAPosts& p, int i, int t0,
+                                              uint64_t smask, uint64_t dmask, int listed0, int listed1)
+{
+    window_append(nd.soma_log, &nd.log_cnt[0], nd.log_cap, smask, i, t0, nd.err);
+    window_append(nd.dend_log, &nd.log_cnt[1], nd.log_cap, dmask, i, t0, nd.err);
+    wl_enlist(nd, 0, smask != 0, listed0, i);
+    wl_enlist(nd, 1, smask != 0, listed1, i);
+    int new_posts = 0;
+    uint64_t pmask = 0;
+    if (p.growth) {
+        for (uint64_t m = smask; m; m &= m - 1) {
+            const int t = t0 + __ffsll((unsigned long long)m) - 1;
+            if (p.count == 0 || win.clk(t) > p.last + 30.0) pmask |= 1ull << (t - t0);
+        }
+    }
+    for (;;) {
+        const bool pred = pmask != 0;
+        const uint64_t b = __ballot(pred);
+        if (b == 0) break;
+        const int lane = __lane_id(), lead = __ffsll((unsigned long long)b) - 1;
+        int base = 0;
+        if (lane == lead) base = atomicAdd(nd.post_list_cnt, __popcll(b));
+        base = __shfl(base, lead);
+        if (pred) {
+            const int t = t0 + __ffsll((unsigned long long)pmask) - 1;
+            const int pos = base + __popcll(b & ((1ull << lane) - 1ull));
+            if (pos < kPostListCap)
+                nd.post_list[pos] = post_key(nd.ra_net[i], t, i);
+            else
+                atomicOr(nd.err, (unsigned)kErrPostList);
+            ++new_posts;
+        }
+        pmask &= pmask - 1;
+    }
+    return new_posts;
+}
+
 // HVC-RA neurons: one thread per neuron (LANES false, `slot` = neuron index) or,
-// RK4 form, four lanes per neuron (LANES true, `slot` = wave index; the quad's
+// RK4 model in the FP32 form, four lanes per neuron (LANES true, `slot` = wave index; the quad's
 // first lane does the neuron's logging and stores)
 template <int MODEL, bool LANES>
 __device__ void integrate_ra(const NetDev& nd, const Win& win, int slot, int t0, int t1)
@@ -407,11 +475,16 @@ __device__ void integrate_ra(const NetDev& nd, const Win& win, int slot, int t0,
     const int lane = LANES ? __lane_id() : 0;
     const int i = LANES ? slot * kRANeuronsPerWave + (lane >> 2) : slot;
     const bool leader = !LANES || (lane & 3) == 0;
+#ifdef HVC_FP32
     RAGateSlot gs[2];
     if (LANES) {
         gs[0] = kRAGates[2 * (lane & 3)];
         gs[1] = kRAGates[2 * (lane & 3) + 1];
     }
+#else
+    static_assert(!LANES, "four lanes per neuron: FP32 form");
+    const int* gs = nullptr;
+#endif
     const bool live = i < nd.n_ra && (!nd.net_live || nd.net_live[nd.ra_net[i]]);
     const int ii = live ? i : 0;
     const int growth = nd.net_growth[nd.ra_net[ii]];
@@ -439,24 +512,7 @@ __device__ void integrate_ra(const NetDev& nd, const Win& win, int slot, int t0,
     const real el = (real)nd.EL[ii], gca = (real)nd.GCa[ii];
     const int kick = nd.kick_step[ii];
 
-    // post events detected in the previous window become visible now (NGS:9385-9386)
-    int pcnt = nd.post_cnt[ii];
-    double last_post = 0.0;
-    if (growth && live && leader) {
-        int pend = nd.post_pend[ii];
-        if (pend > 0) {
-            double cs = win.clk(t0 - 1);
-            for (int q = 0; q < pend; ++q) {
-                nd.post_ring[(size_t)ii * kPostRing + (pcnt % kPostRing)] = cs;
-                ++pcnt;
-            }
-            if (pend > 2) atomicOr(nd.err, (unsigned)kErrPostRing);
-            nd.post_cnt[ii] = pcnt;
-            nd.post_pend[ii] = 0;
-        }
-        if (pcnt > 0) last_post = nd.post_ring[(size_t)ii * kPostRing + ((pcnt - 1) % kPostRing)];
-    }
-    int new_posts = 0;
+    const RAPosts posts = ra_posts_begin(nd, win, growth, ii, t0, live && leader);
 
     const NoiseId sid = ra_noise_id(nd, ii);
     NoiseCursor nc;
@@ -491,39 +547,7 @@ __device__ void integrate_ra(const NetDev& nd, const Win& win, int slot, int t0,
         if (soma) smask |= 1ull << (t - t0);
         if (dend) dmask |= 1ull << (t - t0);
     }
-    // after the steps: the spike logs, and the new postsynaptic events (NGS:8956-8967;
-    // a window's events become visible in the next window, so each spike is
-    // tested against the events of earlier windows only, as in the step loop)
-    window_append(nd.soma_log, &nd.log_cnt[0], nd.log_cap, smask, i, t0, nd.err);
-    window_append(nd.dend_log, &nd.log_cnt[1], nd.log_cap, dmask, i, t0, nd.err);
-    wl_enlist(nd, 0, smask != 0, listed0, i);
-    wl_enlist(nd, 1, smask != 0, listed1, i);
-    uint64_t pmask = 0;
-    if (growth) {
-        for (uint64_t m = smask; m; m &= m - 1) {
-            const int t = t0 + __ffsll((unsigned long long)m) - 1;
-            if (pcnt == 0 || win.clk(t) > last_post + 30.0) pmask |= 1ull << (t - t0);
-        }
-    }
-    for (;;) {
-        const bool pred = pmask != 0;
-        const uint64_t b = __ballot(pred);
-        if (b == 0) break;
-        const int lane = __lane_id(), lead = __ffsll((unsigned long long)b) - 1;
-        int base = 0;
-        if (lane == lead) base = atomicAdd(nd.post_list_cnt, __popcll(b));
-        base = __shfl(base, lead);
-        if (pred) {
-            const int t = t0 + __ffsll((unsigned long long)pmask) - 1;
-            const int pos = base + __popcll(b & ((1ull << lane) - 1ull));
-            if (pos < kPostListCap)
-                nd.post_list[pos] = post_key(nd.ra_net[i], t, i);
-            else
-                atomicOr(nd.err, (unsigned)kErrPostList);
-            ++new_posts;
-        }
-        pmask &= pmask - 1;
-    }
+    const int new_posts = ra_window_logs(nd, win, posts, i, t0, smask, dmask, listed0, listed1);
     if (live && leader) {
         nd.ra[0][i] = HVC_WIDE(s, Vs); nd.ra[1][i] = HVC_WIDE(s, Vd); nd.ra[2][i] = HVC_WIDE(s, n);
         nd.ra[3][i] = HVC_WIDE(s, l); nd.ra[4][i] = HVC_WIDE(s, h); nd.ra[5][i] = HVC_WIDE(s, r);
@@ -585,6 +609,7 @@ __device__ void integrate_i_thread(const NetDev& nd, const Win& win, int i, int 
     }
 }
 
+#ifdef HVC_FP32
 constexpr int kILanes = 5;                    // lanes per HVC-I neuron (DP8)
 constexpr int kINeuronsPerWave = 64 / kILanes; // 12 neurons, 4 idle lanes
 
@@ -726,8 +751,11 @@ __device__ void integrate_i_quad(const NetDev& nd, const Win& win, int wave, int
     }
 }
 
+#endif  // HVC_FP32
+
 constexpr int kINeuronsPerOctWave = 8;       // eight lanes per HVC-I neuron
 
+#ifdef HVC_FP32
 // HVC-I, eight lanes per neuron (DP8 form); one wave holds 8 neurons
 __device__ void integrate_i_oct(const NetDev& nd, const Win& win, int wave, int t0, int t1)
 {
@@ -761,9 +789,7 @@ __device__ void integrate_i_oct(const NetDev& nd, const Win& win, int wave, int 
         nc.none();
     real xo = var == 0 ? s.V : (var == 1 ? s.n : (var == 2 ? s.m : (var == 3 ? s.h : s.w)));
     real xlo = 0;
-#ifdef HVC_FP32
     xlo = var == 0 ? s.V_lo : (var == 1 ? s.n_lo : (var == 2 ? s.m_lo : (var == 3 ? s.h_lo : s.w_lo)));
-#endif
     uint64_t mask = 0;
     for (int t = t0; t <= t1; ++t) {
         int f = i_state_check(s.V, flag);
@@ -780,11 +806,7 @@ __device__ void integrate_i_oct(const NetDev& nd, const Win& win, int wave, int 
     wl_enlist(nd, 2, mask != 0, listed, i);
     if (live && (q < 4 || q == 7)) {
         // lanes 0-3 write V, n, m, h and lane 7 w, widened with their low parts
-#ifdef HVC_FP32
         nd.in[var][i] = (double)xo + (double)xlo;
-#else
-        nd.in[var][i] = xo;
-#endif
     }
     if (live && q == 0) {
         nd.in[5][i] = s.Ge; nd.in[6][i] = s.Gi;
@@ -793,15 +815,190 @@ __device__ void integrate_i_oct(const NetDev& nd, const Win& win, int wave, int 
         nd.i_mask[i] = mask;
     }
 }
+#else
+// the block's tables of the octet steppers
+struct OctLds {
+    ExpPair* exp;       // [64]
+    RANoise* noise;     // [kNoiseRows], Debraband model
+    uint8_t* at;        // 2 kMaxWindowSteps per octet of the block (noise_window)
+};
 
-// blocks [0, iblocks) integrate HVC-I (five lanes per neuron, 12 neurons per
-// wave; four lanes, 16 per wave; or one thread per neuron), the next rblocks
-// HVC-RA (four lanes per neuron, 16 neurons per wave, or one thread per
-// neuron); any blocks after them run the previous window's sync-point STDP
+// one of a neuron's state arrays by lane (selects: an indexed read of the
+// pointers would be a memory round trip of its own)
+template <int N>
+__device__ __forceinline__ double* state_array(double* const (&arrays)[N], int k)
+{
+    double* p = arrays[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j) p = k == j ? arrays[j] : p;
+    return p;
+}
+// HVC-I octet lane -> V n m h w; HVC-RA octet lane -> Vs Vd n l h r c Ca
+__device__ __forceinline__ int i_oct_var(int q) { return q == 0 ? 0 : (q == 7 ? 4 : (q < 4 ? q : 7 - q)); }
+__device__ __forceinline__ int ra_oct_var(int q) { return (int)(0x67153420u >> (4 * q)) & 0xf; }
+
+// HVC-I, eight lanes per neuron (DP8 form); one wave holds 8 neurons
+__device__ void integrate_i_oct(const NetDev& nd, const Win& win, const OctLds& lds, int wave, int t0, int t1)
+{
+    const int lane = __lane_id();
+    const int q = lane & 7;
+    const int i = wave * kINeuronsPerOctWave + (lane >> 3);
+    const bool live = i < nd.n_i && (!nd.net_live || nd.net_live[nd.i_net[i]]);
+    const int ii = live ? i : 0;
+    double* xp = state_array<7>(nd.in, i_oct_var(q));
+    double x = xp[ii];
+    if (q > 3 && q < 7) x = 1 - x;
+    const int listed = nd.wl_on ? nd.wl_mark[2][ii] : 0;
+    double Ge = nd.in[5][ii], Gi = nd.in[6][ii];
+    int flag = nd.i_flag[ii];
+    const IOctLane L = i_oct_lane(q, lds.exp);
+    stage_exp_table(lds.exp);
+    win.stage(nd);
+    // the previous window's sync: HHI raiseE (Ge += G); only the octet's first
+    // lane uses the conductances
+    if (live && q == 0) {
+        double sum;
+        if (inbox_take(nd, nd.in_ge_i, i, sum)) Ge += sum;
+    }
+    NoiseCursor nc;
+    if (nd.i_poisson)
+        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, nd.i_ev_pos[ii]);
+    else
+        nc.none();
+    const double dt = nd.dt;
+    Dp8Consts C;
+    dp8_pin(C);
+    uint64_t mask = 0;
+    for (int t = t0; t <= t1; ++t) {
+        const int f = i_state_check(x, flag);   // of V in lane 0
+        // HHI_buffer noise checks (Ge, Gi), as listed
+        nc.take(t, [&](int gi, double inc) {
+            Ge = gi == 0 ? Ge + inc : Ge;
+            Gi = gi == 1 ? Gi + inc : Gi;
+        });
+        i_oct_step(L, C, x, Ge, Gi, dt, win.row(t));
+        if (live && f && q == 0) mask |= 1ull << (t - t0);
+    }
+    window_append(nd.i_log, &nd.log_cnt[2], nd.log_cap, mask, i, t0, nd.err);
+    wl_enlist(nd, 2, mask != 0, listed, i);
+    if (live && (q < 4 || q == 7)) xp[i] = x;
+    if (live && q == 0) {
+        nd.in[5][i] = Ge; nd.in[6][i] = Gi;
+        nd.i_flag[i] = flag;
+        if (nd.i_poisson) nd.i_ev_pos[i] = nc.pos;
+        nd.i_mask[i] = mask;
+    }
+}
+
+// the spike detection of an HVC-RA octet lane: the soma's in lane 0 (bit 0),
+// the dendrite's in lane 5 (bit 1) (ra_state_check, HH2_test.cpp:561-594)
+__device__ __forceinline__ int ra_oct_check(int q, double x, int& flag)
+{
+    int f = 0;
+    if (q == 0) {
+        if (flag == 1 && x < -30.0 - 5.0) {
+            flag = 0;
+            f = 1;
+        } else if (flag == 0 && x > -30.0) {
+            flag = 1;
+        }
+    } else if (q == 5) {
+        if (flag == 0 && x >= -30.0) {
+            flag = 1;
+            f = 2;
+        } else if (flag == 1 && x < -30.0 - 5.0) {
+            flag = 0;
+        }
+    }
+    return f;
+}
+
+// HVC-RA, eight lanes per neuron; one wave holds 8 neurons.  Lane 0 keeps the
+// neuron's events, lane 5 its dendritic spikes.
+template <int MODEL>
+__device__ void integrate_ra_oct(const NetDev& nd, const Win& win, const OctLds& lds, int wave, int t0, int t1)
+{
+    const int lane = __lane_id();
+    const int q = lane & 7;
+    const int i = wave * kRAOctNeuronsPerWave + (lane >> 3);
+    const bool live = i < nd.n_ra && (!nd.net_live || nd.net_live[nd.ra_net[i]]);
+    const int ii = live ? i : 0;
+    const bool soma = live && q == 0, dend = live && q == 5;
+    const int growth = nd.net_growth[nd.ra_net[ii]];
+    const int listed0 = nd.wl_on ? nd.wl_mark[0][ii] : 0, listed1 = nd.wl_on ? nd.wl_mark[1][ii] : 0;
+    double* xp = state_array<12>(nd.ra, ra_oct_var(q));
+    double x = xp[ii];
+    // the lane's two synaptic conductances (ra_oct_deriv): Gi_s, Ge_s or Ge_d, Gi_d
+    double* const gap = q == 0 ? nd.ra[9] : nd.ra[10];
+    double* const gbp = q == 0 ? nd.ra[8] : nd.ra[11];
+    double GA = gap[ii], GB = gbp[ii];
+    const int flags = nd.ra_flags[ii];
+    int flag = q == 0 ? flags & 1 : (flags >> 1) & 1;
+    const int kick = nd.kick_step[ii];
+    const NoiseId sid = ra_noise_id(nd, ii);
+    const RAOctLane L = ra_oct_lane<MODEL>(q, nd.EL[ii], nd.GCa[ii], nd.mu_term_s, nd.mu_term_d, lds.exp);
+    uint8_t* at = lds.at + (threadIdx.x >> 3) * (2 * kMaxWindowSteps);
+    stage_exp_table(lds.exp);
+    if constexpr (MODEL == 0) {
+        stage_noise_rows(lds.noise, nd.sq_sig_s, nd.sq_sig_d);
+        noise_window(at, q, sid, t0, t1 - t0 + 1);
+    }
+    win.stage(nd);
+    // the previous window's sync: raiseExcWeight (Ge_d += w / Ad), raiseI (Gi_d += G)
+    if (dend) {
+        double sum;
+        if (inbox_take(nd, nd.in_gi_ra, i, sum)) GB += sum;
+        if (inbox_take(nd, nd.in_ge_ra, i, sum)) GA += HVC_CDIV(sum, 10000);
+    }
+    const RAPosts posts = ra_posts_begin(nd, win, growth, ii, t0, soma);
+    NoiseCursor nc;
+    if (MODEL == 1 && nd.ra_poisson)
+        nc.open(nd.ra_ev + (size_t)ii * nd.ev_cap, nd.ra_ev_pos[ii]);
+    else
+        nc.none();
+    const double dt = nd.dt;
+    uint64_t mask = 0;   // somatic spikes in lane 0, dendritic ones in lane 5
+    for (int t = t0; t <= t1; ++t) {
+        if (kick == t && q == 5) GA += 3.0;   // raiseE(G_TRAINING_KICK), NGS:8933-8940
+        const int f = ra_oct_check(q, x, flag);
+        RANoise nz{};
+        if constexpr (MODEL == 0) {
+            const int k = 2 * (t - t0);
+            nz = lds.noise[q == 0 ? at[k] : (q == 5 ? at[k + 1] : kNoiseRows - 1)];
+        } else {
+            // HH2_buffer noise checks (Gi_s, Gi_d, Ge_s, Ge_d), as listed
+            nc.take(t, [&](int g, double inc) {
+                GA = (g == 0 && q == 0) || (g == 3 && q == 5) ? GA + inc : GA;
+                GB = (g == 2 && q == 0) || (g == 1 && q == 5) ? GB + inc : GB;
+            });
+        }
+        ra_oct_step<MODEL>(L, x, GA, GB, dt, nz, win.row(t));
+        if (live && f) mask |= 1ull << (t - t0);
+    }
+    const int new_posts = ra_window_logs(nd, win, posts, i, t0, q == 0 ? mask : 0, q == 5 ? mask : 0, listed0, listed1);
+    const int fd = __shfl(flag, (lane & ~7) + 5);
+    if (live && (MODEL == 0 || q != 3)) xp[i] = x;
+    if (soma || dend) {
+        gap[i] = GA;
+        gbp[i] = GB;
+        (soma ? nd.soma_mask : nd.dend_mask)[i] = mask;
+    }
+    if (soma) {
+        nd.ra_flags[i] = flag | (fd << 1);
+        if (growth) nd.post_pend[i] = new_posts;
+        if (MODEL == 1 && nd.ra_poisson) nd.ra_ev_pos[i] = nc.pos;
+    }
+}
+#endif
+
+// blocks [0, iblocks) integrate HVC-I, the next rblocks HVC-RA, in the layout
+// of LANES; any blocks after them run the previous window's sync-point STDP
 // (one row per thread, sa).
-// LANES: bit 0 = HVC-I five lanes, bit 1 = HVC-RA four lanes, bit 2 = HVC-I
-// four lanes, bit 3 = HVC-I eight lanes (the layouts are template parameters: a
-// kernel holds the register allocation of one layout only)
+// LANES: HVC-I bit 0 = five lanes, bit 2 = four lanes, bit 3 = eight lanes per
+// neuron, none = one thread; HVC-RA bit 1 = four lanes (FP32 form) or eight
+// (FP64 form), else one thread.  (The layouts are template parameters: a
+// kernel holds the register allocation of one layout only.  The FP64 form has
+// the octets and one thread.)
 template <int RA_MODEL, int I_MODEL, int LANES>
 __global__ __launch_bounds__(256) void k_integrate(NetDev nd, int t0, int t1, int iblocks, int rblocks, StdpArgs sa)
 {
@@ -816,28 +1013,58 @@ __global__ __launch_bounds__(256) void k_integrate(NetDev nd, int t0, int t1, in
     extern __shared__ double win_lds[];
     const int nsteps = t1 - t0 + 1;
     const Win win{(const WinRow*)win_lds, (const double*)((const WinRow*)win_lds + nsteps), t0, win_lds, nsteps};
+    const int iwave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int rwave = (blockIdx.x - iblocks) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+#ifdef HVC_FP32
     if ((int)blockIdx.x < iblocks) {
         if constexpr ((LANES & 8) != 0)
-            integrate_i_oct(nd, win, blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), t0, t1);
+            integrate_i_oct(nd, win, iwave, t0, t1);
         else if constexpr ((LANES & 4) != 0)
-            integrate_i_quad(nd, win, blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), t0, t1);
+            integrate_i_quad(nd, win, iwave, t0, t1);
         else if constexpr ((LANES & 1) != 0)
-            integrate_i_lanes(nd, win, blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), t0, t1);
+            integrate_i_lanes(nd, win, iwave, t0, t1);
         else
             integrate_i_thread<I_MODEL>(nd, win, blockIdx.x * blockDim.x + threadIdx.x, t0, t1);
     } else {
         if constexpr ((LANES & 2) != 0)
-            integrate_ra<RA_MODEL, true>(nd, win, (blockIdx.x - iblocks) * (blockDim.x >> 6) + (threadIdx.x >> 6),
-                                         t0, t1);
+            integrate_ra<RA_MODEL, true>(nd, win, rwave, t0, t1);
         else
             integrate_ra<RA_MODEL, false>(nd, win, (blockIdx.x - iblocks) * blockDim.x + threadIdx.x, t0, t1);
     }
+#else
+    __shared__ ExpPair exp_tab[64];
+    __shared__ RANoise noise_rows[RA_MODEL == 0 && (LANES & 2) ? kNoiseRows : 1];
+    __shared__ uint8_t noise_at[RA_MODEL == 0 && (LANES & 2) ? 256 / 8 * 2 * kMaxWindowSteps : 1];
+    const OctLds lds{exp_tab, noise_rows, noise_at};
+    if ((int)blockIdx.x < iblocks) {
+        if constexpr ((LANES & 8) != 0)
+            integrate_i_oct(nd, win, lds, iwave, t0, t1);
+        else
+            integrate_i_thread<I_MODEL>(nd, win, blockIdx.x * blockDim.x + threadIdx.x, t0, t1);
+    } else {
+        if constexpr ((LANES & 2) != 0)
+            integrate_ra_oct<RA_MODEL>(nd, win, lds, rwave, t0, t1);
+        else
+            integrate_ra<RA_MODEL, false>(nd, win, (blockIdx.x - iblocks) * blockDim.x + threadIdx.x, t0, t1);
+    }
+#endif
 }
 
 // LDS bytes of k_integrate for a window of n steps
 static inline size_t win_bytes(int n) { return (size_t)n * sizeof(WinRow) + (size_t)(n + 1) * sizeof(double); }
 
 }  // namespace p32 / p64
+
+#ifndef HVC_FP32
+// HVC-RA neurons per context up to which a window takes octets without being
+// asked.  An octet's wave is short (640 instructions per Debraband step, the
+// one-thread wave 5 600 before the two-operation quotients, 4 700 with them)
+// but eight times as many are needed.  k_integrate per window beside HVC-I
+// octets (n / 3.6 of them), octets / one thread, us: Debraband 82 / 98 at
+// 20 000 neurons, 106 / 116 at 30 000, 134 / 117 at 40 000; RK4 76 / 82 at
+// 20 000, 99 / 99 at 30 000, 126 / 99 at 40 000.
+constexpr int kRAOctMaxNeurons[2] = {32768, 16384};   // by ra_model
+#endif
 
 #ifdef HVC_FP32
 #define HVC_LAUNCHER(name) name##_f32
@@ -862,19 +1089,32 @@ void HVC_LAUNCHER(launch_integrate)(hipStream_t st, const NetDev& nd, int t0, in
                                      const StdpArgs& sa, int stdp)
 {
     const int bs = tu.integrate_block;
+    const int wpb = bs / 64;
+#ifdef HVC_FP32
     // HVC-I layout (DP8 only): 0 one thread, 1 five lanes, 2 four lanes, 3 eight lanes per neuron
     const int i_layout = nd.i_model == 0 ? tu.i_lanes : 0;
     const int ra_lanes = (nd.ra_model == 1 && tu.ra_lanes) ? 1 : 0;
-    const int i_per_block = i_layout == 1 ? (bs / 64) * kINeuronsPerWave
-                            : (i_layout == 2 ? (bs / 64) * kINeuronsPerQuadWave
-                                             : (i_layout == 3 ? (bs / 64) * kINeuronsPerOctWave : bs));
-    const int ra_per_block = ra_lanes ? (bs / 64) * kRANeuronsPerWave : bs;
+    const int ra_per_block = ra_lanes ? wpb * kRANeuronsPerWave : bs;
+    const int i_per_block = i_layout == 1 ? wpb * kINeuronsPerWave
+                            : (i_layout == 2 ? wpb * kINeuronsPerQuadWave
+                                             : (i_layout == 3 ? wpb * kINeuronsPerOctWave : bs));
+#else
+    // the FP64 layouts give the same bits, so every HVC-I layout with several
+    // lanes is the octet (45 us per window at 2 000 + 550 neurons; the four-lane
+    // and the earlier eight-lane form took 84 and 67 us), and HVC-RA takes
+    // octets when asked to or when the network is small enough
+    const int i_layout = nd.i_model == 0 && tu.i_lanes ? 3 : 0;
+    const int ra_lanes = tu.ra_lanes || nd.n_ra <= kRAOctMaxNeurons[nd.ra_model == 1];
+    const int ra_per_block = ra_lanes ? wpb * kRAOctNeuronsPerWave : bs;
+    const int i_per_block = i_layout ? wpb * kINeuronsPerOctWave : bs;
+#endif
     int iblocks = nd.n_i == 0 ? 0 : (nd.n_i + i_per_block - 1) / i_per_block;
     int rblocks = blocks_for(nd.n_ra, ra_per_block);
     const int sblocks = stdp ? blocks_for(nd.n_ra, bs) : 0;
     dim3 grid(iblocks + rblocks + sblocks);
     const size_t lds = win_bytes(t1 - t0 + 1);
 #define HVC_K(R, I, L) k_integrate<R, I, L><<<grid, bs, lds, st>>>(nd, t0, t1, iblocks, rblocks, sa)
+#ifdef HVC_FP32
     if (nd.ra_model == 0) {
         if (nd.i_model == 1) HVC_K(0, 1, 0);
         else if (i_layout == 3) HVC_K(0, 0, 8);
@@ -894,6 +1134,25 @@ void HVC_LAUNCHER(launch_integrate)(hipStream_t st, const NetDev& nd, int t0, in
         else if (i_layout == 1) HVC_K(1, 0, 1);
         else HVC_K(1, 0, 0);
     }
+#else
+#define HVC_KR(R)                              \
+    if (nd.i_model == 1) {                     \
+        if (ra_lanes) HVC_K(R, 1, 2);          \
+        else HVC_K(R, 1, 0);                   \
+    } else if (i_layout) {                     \
+        if (ra_lanes) HVC_K(R, 0, 10);         \
+        else HVC_K(R, 0, 8);                   \
+    } else {                                   \
+        if (ra_lanes) HVC_K(R, 0, 2);          \
+        else HVC_K(R, 0, 0);                   \
+    }
+    if (nd.ra_model == 0) {
+        HVC_KR(0)
+    } else {
+        HVC_KR(1)
+    }
+#undef HVC_KR
+#endif
 #undef HVC_K
 }
 

@@ -53,17 +53,18 @@ __device__ __forceinline__ double dexp(double x)
     return __builtin_ldexp(y, e);  // v_ldexp_f64: one rounding, also for subnormal results
 }
 
-// a / B for a divisor B > 0 known at compile time, with Y = RN(1/B): q = RN(a Y),
-// r = a - B q (exact, fma), result RN(q + r Y) -- Markstein's correction
-// (Markstein 1990, IBM J. Res. Dev. 34(1)).  For 2^-900 <= |q| < 2^1000:
-// |q - a/B| < 1.5 ulp, r is exact, and the fma result differs from a/B by at
-// most 3 * 2^-54 ulp while a/B lies at least ulp / (4 B_odd) from every
-// rounding boundary (B_odd = odd part of B's significand); for B_odd < 2^51 --
-// every divisor used here -- the result is the correctly rounded quotient, bit
-// for bit a / B.  For a = +-0 the result is a zero with a's sign, as a / B is.
-// Any other quotient (tiny, huge, infinite or NaN) is recorded in the guard and
-// the caller repeats the step with IEEE division.  No branch, so the compiler
-// can interleave the many independent quotients of a stage.
+// a / B for a divisor B known at compile time, as RN(a Yh + RN(a Yl)) with Yh =
+// RN(1/B) and Yl = RN(1/B - Yh) (Brisebarre, Muller, Raina 2004, IEEE Trans.
+// Comput. 53(8)): one multiplication and one fma.  For 2^-900 <= |a/B| <
+// 2^1000 the sum before its rounding differs from a/B by at most 2^-105 |a/B|
+// (2^-106 from Yl, 2^-106 from the product's rounding), under 2^-52 ulp, while
+// a/B lies at least ulp / (4 B_odd) from every rounding boundary (B_odd = odd
+// part of B's significand); for B_odd < 2^49 -- every divisor used here -- the
+// result is the correctly rounded quotient, bit for bit a / B but for the
+// sign of a zero.  Any other quotient (tiny, huge, infinite or NaN) is
+// recorded in the guard and the caller repeats the step with IEEE division.
+// No branch, so the compiler can interleave the many independent quotients of
+// a stage.
 struct DivGuard {
     int emin = 0;      // least binary exponent of a quotient (frexp convention, 0 for zero)
     double big = 0.0;  // sum of |q| 2^-1000: >= 1 or NaN once a quotient is huge or not finite
@@ -72,37 +73,27 @@ struct DivGuard {
         emin = min(emin, __builtin_amdgcn_frexp_exp(q));
         big = __builtin_fma(__builtin_fabs(q), 0x1p-1000, big);
     }
-    // a value k that enters tableau terms (n k) / d with n / d in [2^-7, 2^5]
-    // and |n| < 2^36 only (DP8 stages 7-12 and the final combination): noting
-    // k once stands for noting each such quotient.  k = 0 or 2^-892 <= |k| <
-    // 2^985 keeps n k finite and every quotient in [2^-899, 2^990) or zero.
-    __device__ __forceinline__ void note_k(double k)
-    {
-        emin = min(emin, __builtin_amdgcn_frexp_exp(k) - 8);
-        big = __builtin_fma(__builtin_fabs(k), 0x1p-985, big);
-    }
     __device__ __forceinline__ bool failed() const { return emin < -899 || !(big < 1.0); }
 };
 
-// Markstein's correction with the rounded reciprocal Y = RN(1 / B)
-__device__ __forceinline__ double cdiv_plain(double a, double B, double Y)
+__device__ __forceinline__ double cdiv2(double a, double B)
 {
-    double q = a * Y;
-    double r = __builtin_fma(-q, B, a);
-    return __builtin_copysign(__builtin_fma(r, Y, q), a);
+    const double Yh = 1.0 / B, Yl = __builtin_fma(-B, Yh, 1.0) / B;   // folded for a literal B
+    return __builtin_fma(a, Yh, a * Yl);
 }
 
-__device__ __forceinline__ double cdiv_fast(double a, double B, double Y, DivGuard& g)
+__device__ __forceinline__ double cdiv_fast(double a, double B, DivGuard& g)
 {
-    g.note(a * Y);
-    return cdiv_plain(a, B, Y);
+    const double q = cdiv2(a, B);
+    g.note(q);
+    return q;
 }
 
 // the same quotient with the IEEE fallback applied per value
 __device__ __forceinline__ double cdiv_checked(double a, double B)
 {
     DivGuard g;
-    double q = cdiv_fast(a, B, 1.0 / B, g);
+    const double q = __builtin_copysign(cdiv_fast(a, B, g), a);
     return g.failed() ? a / B : q;
 }
 #define HVC_CDIV(a, B) ::hvc::cdiv_checked((a), (double)(B))

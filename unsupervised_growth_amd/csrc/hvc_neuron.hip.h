@@ -38,13 +38,10 @@ typedef float real;
 struct Guard {
     static constexpr bool kActive = false;
     __device__ __forceinline__ bool failed() const { return false; }
-    __device__ __forceinline__ void note_k(real) const {}
 };
 #define HR(x) ((real)(x))
 #define CD(a, B) ((a) * (real)(1.0 / (double)(B)))
-#define CDV(a, B, invB) ((a) * (invB))
 #define CK(n, k, d) ((k) * (real)((double)(n) / (double)(d)))
-#define CKN(n, k, d) CK(n, k, d)
 #define DIVR(a, b) ((real)(a) * __builtin_amdgcn_rcpf((real)(b)))
 // exp(a / B) as 2^(a * RN(log2(e) / B)): the argument a / B is already only
 // known to |a / B| * 2^-24 in this form, and folding log2(e) into the constant
@@ -74,21 +71,20 @@ struct Guard : DivGuard {
 };
 #define HR(x) ((real)(x))
 // constant-divisor quotient inside a stepper: IEEE division when EXACT, else the
-// branch-free Markstein form, whose guard `bad` tells when the step must be repeated
-#define CD(a, B) (EXACT ? (a) / (double)(B) : ::hvc::cdiv_fast((a), (double)(B), 1.0 / (double)(B), bad))
-#define CDV(a, B, invB) (EXACT ? (a) / (B) : ::hvc::cdiv_fast((a), (B), (invB), bad))
+// branch-free form, whose guard `bad` tells when the step must be repeated
+#define CD(a, B) (EXACT ? (a) / (double)(B) : ::hvc::cdiv_fast((a), (double)(B), bad))
 // tableau term (n k) / d, evaluated as the reference writes it
 #define CK(n, k, d) CD((n) * (k), d)
-// the same term for a k the step notes itself (DivGuard::note_k)
-#define CKN(n, k, d) (EXACT ? ((n) * (k)) / (double)(d) : ::hvc::cdiv_plain((n) * (k), (double)(d), 1.0 / (double)(d)))
 #define DIVR(a, b) ((a) / (b))
 #define EXPR(x) ::hvc::dexp(x)
 #define EXPCD(a, B) EXPR(CD(a, B))
-#define EXPCDV(a, B, invB, inv2B) EXPR(CDV(a, B, invB))
 #define HVC_FP_FAST
 #define HVC_KEEP(x)
 #define HVC_ACC(st, f, inc) st.f = st.f + inc;
 #endif
+
+// RN(log2(e) / e) of a gate's e
+#define HVC_L2(e) (real)(1.4426950408889634 / (e))
 
 // offsets c*dt of the stage times used by the steppers, in this order
 enum DecayOffset {
@@ -312,7 +308,8 @@ __device__ __forceinline__ RAK ra_rhs(Guard& bad, const RAState& s, real EL, rea
 #endif
 }
 
-// ---- HVC-RA, RK4 form, four lanes per neuron ----
+// ---- HVC-RA, RK4 form, four lanes per neuron (FP32 form; FP64: hvc_oct64.hip.h) ----
+#ifdef HVC_FP32
 // The seven gates of HH2_buffer share one form, a + c / (1 + exp(+-(v + d) / e))
 // on Vs or Vd.  Lane q of a neuron's quad evaluates gate slots 2q and 2q + 1,
 // DPP quad broadcasts hand every lane all seven, and every lane then evaluates
@@ -325,7 +322,6 @@ struct RAGateSlot {
 };
 
 __constant__ RAGateSlot kRAGates[8] = {
-#define HVC_L2(e) (real)(1.4426950408889634 / (e))
     {HR(0.0), HR(1.0), HR(30.0), HR(9.5), (real)(1.0 / 9.5), 1, 0, HVC_L2(9.5)},     // mInf
     {HR(0.0), HR(1.0), HR(35.0), HR(10.0), (real)(1.0 / 10.0), 1, 0, HVC_L2(10.0)},  // nInf
     {HR(0.1), HR(0.5), HR(27.0), HR(15.0), (real)(1.0 / 15.0), 0, 0, HVC_L2(15.0)},  // tauN
@@ -344,6 +340,7 @@ __device__ __forceinline__ real ra_gate(Guard& bad, const RAGateSlot& g, real vs
     real q = DIVR(g.c, 1 + EXPCDV(g.neg ? -x : x, g.e, g.inv_e, g.inv2_e));
     return g.a + q;   // a = 0: 0 + q = q (q > 0)
 }
+#endif
 
 // value of lane K of the quad, in every lane of the quad (DPP quad_perm)
 template <int K>
@@ -360,13 +357,14 @@ __device__ __forceinline__ double quad_bcast(double x)
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-template <bool EXACT, bool LANES>
+template <bool EXACT, bool LANES, class Slot>
 __device__ __forceinline__ RAK ra_rhs4(Guard& bad, const RAState& s, real EL, real GCa, const RAUniform& u,
-                                       const RAGateSlot* sl, real vs, real vd, real n, real h, real r, real c,
+                                       const Slot* sl, real vs, real vd, real n, real h, real r, real c,
                                        real ca, real E)
 {
-    RAGates g;
+#ifdef HVC_FP32
     if constexpr (LANES) {
+        RAGates g;
         const real g0 = ra_gate<EXACT>(bad, sl[0], vs, vd);
         const real g1 = ra_gate<EXACT>(bad, sl[1], vs, vd);
         g.m = quad_bcast<0>(g0);
@@ -377,15 +375,14 @@ __device__ __forceinline__ RAK ra_rhs4(Guard& bad, const RAState& s, real EL, re
         g.rI = quad_bcast<2>(g1);
         g.cI = quad_bcast<3>(g0);
         g.lI = HR(0.0);
-    } else {
-#ifdef HVC_FP32
+        return ra_rhs_g<1, EXACT>(bad, s, EL, GCa, u, g, vs, vd, n, h, HR(0.0), r, c, ca, E);
+    } else
         return ra_rhs_g<1, EXACT, true>(bad, s, EL, GCa, u, ra_gates<1, EXACT, true>(bad, vs, vd), vs, vd, n, h,
                                         HR(0.0), r, c, ca, E);
 #else
-        g = ra_gates<1, EXACT>(bad, vs, vd);
+    static_assert(!LANES, "four lanes per neuron: FP32 form");
+    return ra_rhs_g<1, EXACT>(bad, s, EL, GCa, u, ra_gates<1, EXACT>(bad, vs, vd), vs, vd, n, h, HR(0.0), r, c, ca, E);
 #endif
-    }
-    return ra_rhs_g<1, EXACT>(bad, s, EL, GCa, u, g, vs, vd, n, h, HR(0.0), r, c, ca, E);
 }
 
 // HH2_test::Debraband_step; J* are the point-distribution values of this step
@@ -438,9 +435,9 @@ __device__ __forceinline__ void ra_debraband(Guard& bad, RAState& s, real EL, re
 }
 
 // HH2_buffer::Runge4_step (Kutta 3/8 rule); LANES: four lanes per neuron, sl = this lane's two gate slots
-template <bool EXACT, bool LANES>
+template <bool EXACT, bool LANES, class Slot>
 __device__ __forceinline__ void ra_runge4(Guard& bad, RAState& s, real EL, real GCa, const RAUniform& u,
-                                          const RAGateSlot* sl, real E_third, real E_twothird, real E_dt)
+                                          const Slot* sl, real E_third, real E_twothird, real E_dt)
 {
     HVC_FP_FAST
     const real dt = u.dt;
@@ -817,14 +814,8 @@ __constant__ real kPointDistribution[30] = {
 
 
 
-// ---------------- HVC-I, five lanes per neuron ----------------
-// DP8 spends its time in the gate rates (7 exp per stage) and in the stage
-// combinations (one per state variable, up to 9 quotients each).  Lane role
-// r = lane % 5 owns variable r of (V, n, m, h, w): it evaluates that variable's
-// gate rates and its combination, and the five stage values are exchanged with
-// cross-lane shuffles.  Every lane evaluates exactly the expression trees of
-// HHI_buffer (HHI_buffer.cpp:426-691, 741-747), so results equal i_dp8 bit for
-// bit.  Rate forms: A = c (v+d) / (1 - E), B = c E, C = c / (1 + E), with
+// ---------------- HVC-I, several lanes per neuron ----------------
+// Rate forms: A = c (v+d) / (1 - E), B = c E, C = c / (1 + E), with
 // E = exp(-(v+d)/e):  an, am: A;  bn, bm, ah: B;  bh, wInf: C.
 struct GateSlot {
     int type;        // 0: A, 1: B, 2: C
@@ -832,6 +823,14 @@ struct GateSlot {
     real inv2_e;     // RN(log2(e) / e) (FP32 form, EXPCDV)
 };
 
+#ifdef HVC_FP32
+// ---- five lanes per neuron ----
+// DP8 spends its time in the gate rates (7 exp per stage) and in the stage
+// combinations (one per state variable, up to 9 quotients each).  Lane role
+// r = lane % 5 owns variable r of (V, n, m, h, w): it evaluates that variable's
+// gate rates and its combination, and the five stage values are exchanged with
+// cross-lane shuffles.  (The FP64 form has one layout with several lanes, the
+// octet of hvc_oct64.hip.h.)
 template <bool EXACT, bool CAN_A = true>
 __device__ __forceinline__ real gate_rate(Guard& bad, const GateSlot& g, real v)
 {
@@ -842,7 +841,6 @@ __device__ __forceinline__ real gate_rate(Guard& bad, const GateSlot& g, real v)
     real den = (g.type == 0) ? (1 - E) : (1 + E);
     real q = DIVR(num, den);
     HVC_KEEP(q);
-#ifdef HVC_FP32
     // form A near v = -d: the series (as rates_vd_near)
     if constexpr (CAN_A) {
         const bool near = g.type == 0 && __builtin_fabsf(vd) <= HR(0.5) * g.e;
@@ -851,7 +849,6 @@ __device__ __forceinline__ real gate_rate(Guard& bad, const GateSlot& g, real v)
             if (near) q = sr;
         }
     }
-#endif
     return (g.type == 1) ? g.c * E : q;
 }
 
@@ -885,40 +882,37 @@ __device__ __forceinline__ real i_lane_rhs(Guard& bad, const IState& s, int role
 }
 
 // DP8 stage values: the combination of stage derivatives P1.. of one
-// variable (HHI_buffer.cpp:426-691), shared by the five-lane and quad forms;
-// the tableau terms of stages 7-12 and the final combination are HVC_CKX
-// (CK, or CKN where the step notes each stage derivative itself)
-#define HVC_CKX CK
+// variable (HHI_buffer.cpp:426-691), shared by the layouts
 #define HVC_DP8_S2(P) HVC_F2(P##1)
 #define HVC_DP8_S3(P) HVC_F3(P##1 + 3 * P##2)
 #define HVC_DP8_S4(P) HVC_F4(P##1 + 3 * P##3)
 #define HVC_DP8_S5(P) HVC_F5(20 * P##1 - 75 * P##3 + 75 * P##4)
 #define HVC_DP8_S6(P) HVC_F6(3 * P##1 + 15 * P##4 + 12 * P##5)
-#define HVC_DP8_S7(P) dt * (HVC_CKX(29443841, P##1, 614563906) + HVC_CKX(77736538, P##4, 692538347) - \
-                            HVC_CKX(28693883, P##5, 1125000000) + HVC_CKX(23124283, P##6, 1800000000))
-#define HVC_DP8_S8(P) dt * (HVC_CKX(16016141, P##1, 946692911) + HVC_CKX(61564180, P##4, 158732637) + \
-                            HVC_CKX(22789713, P##5, 633445777) + HVC_CKX(545815736, P##6, 2771057229) - \
-                            HVC_CKX(180193667, P##7, 1043307555))
-#define HVC_DP8_S9(P) dt * (HVC_CKX(39632708, P##1, 573591083) - HVC_CKX(433636366, P##4, 683701615) - \
-                            HVC_CKX(421739975, P##5, 2616292301) + HVC_CKX(100302831, P##6, 723423059) + \
-                            HVC_CKX(790204164, P##7, 839813087) + HVC_CKX(800635310, P##8, 3783071287))
-#define HVC_DP8_S10(P) dt * (HVC_CKX(246121993, P##1, 1340847787) - HVC_CKX(37695042795, P##4, 15268766246) - \
-                             HVC_CKX(309121744, P##5, 1061227803) - HVC_CKX(12992083, P##6, 490766935) + \
-                             HVC_CKX(6005943493, P##7, 2108947869) + HVC_CKX(393006217, P##8, 1396673457) + \
-                             HVC_CKX(123872331, P##9, 1001029789))
-#define HVC_DP8_S11(P) dt * (HVC_CKX(-1028468189, P##1, 846180014) + HVC_CKX(8478235783, P##4, 508512852) + \
-                             HVC_CKX(1311729495, P##5, 1432422823) - HVC_CKX(10304129995, P##6, 1701304382) - \
-                             HVC_CKX(48777925059, P##7, 3047939560) + HVC_CKX(15336726248, P##8, 1032824649) - \
-                             HVC_CKX(45442868181, P##9, 3398467696) + HVC_CKX(3065993473, P##10, 597172653))
-#define HVC_DP8_S12(P) dt * (HVC_CKX(185892177, P##1, 718116043) - HVC_CKX(3185094517, P##4, 667107341) - \
-                             HVC_CKX(477755414, P##5, 1098053517) - HVC_CKX(703635378, P##6, 230739211) + \
-                             HVC_CKX(5731566787, P##7, 1027545527) + HVC_CKX(5232866602, P##8, 850066563) - \
-                             HVC_CKX(4093664535, P##9, 808688257) + HVC_CKX(3962137247, P##10, 1805957418) + \
-                             HVC_CKX(65686358, P##11, 487910083))
-#define HVC_DP8_FIN(P) dt * (HVC_CKX(13451932, P##1, 455176623) - HVC_CKX(808719846, P##6, 976000145) + \
-                             HVC_CKX(1757004468, P##7, 5645159321) + HVC_CKX(656045339, P##8, 265891186) - \
-                             HVC_CKX(3867574721, P##9, 1518517206) + HVC_CKX(465885868, P##10, 322736535) + \
-                             HVC_CKX(53011238, P##11, 667516719) + HVC_CKX(2, P##12, 45))
+#define HVC_DP8_S7(P) dt * (CK(29443841, P##1, 614563906) + CK(77736538, P##4, 692538347) - \
+                            CK(28693883, P##5, 1125000000) + CK(23124283, P##6, 1800000000))
+#define HVC_DP8_S8(P) dt * (CK(16016141, P##1, 946692911) + CK(61564180, P##4, 158732637) + \
+                            CK(22789713, P##5, 633445777) + CK(545815736, P##6, 2771057229) - \
+                            CK(180193667, P##7, 1043307555))
+#define HVC_DP8_S9(P) dt * (CK(39632708, P##1, 573591083) - CK(433636366, P##4, 683701615) - \
+                            CK(421739975, P##5, 2616292301) + CK(100302831, P##6, 723423059) + \
+                            CK(790204164, P##7, 839813087) + CK(800635310, P##8, 3783071287))
+#define HVC_DP8_S10(P) dt * (CK(246121993, P##1, 1340847787) - CK(37695042795, P##4, 15268766246) - \
+                             CK(309121744, P##5, 1061227803) - CK(12992083, P##6, 490766935) + \
+                             CK(6005943493, P##7, 2108947869) + CK(393006217, P##8, 1396673457) + \
+                             CK(123872331, P##9, 1001029789))
+#define HVC_DP8_S11(P) dt * (CK(-1028468189, P##1, 846180014) + CK(8478235783, P##4, 508512852) + \
+                             CK(1311729495, P##5, 1432422823) - CK(10304129995, P##6, 1701304382) - \
+                             CK(48777925059, P##7, 3047939560) + CK(15336726248, P##8, 1032824649) - \
+                             CK(45442868181, P##9, 3398467696) + CK(3065993473, P##10, 597172653))
+#define HVC_DP8_S12(P) dt * (CK(185892177, P##1, 718116043) - CK(3185094517, P##4, 667107341) - \
+                             CK(477755414, P##5, 1098053517) - CK(703635378, P##6, 230739211) + \
+                             CK(5731566787, P##7, 1027545527) + CK(5232866602, P##8, 850066563) - \
+                             CK(4093664535, P##9, 808688257) + CK(3962137247, P##10, 1805957418) + \
+                             CK(65686358, P##11, 487910083))
+#define HVC_DP8_FIN(P) dt * (CK(13451932, P##1, 455176623) - CK(808719846, P##6, 976000145) + \
+                             CK(1757004468, P##7, 5645159321) + CK(656045339, P##8, 265891186) - \
+                             CK(3867574721, P##9, 1518517206) + CK(465885868, P##10, 322736535) + \
+                             CK(53011238, P##11, 667516719) + CK(2, P##12, 45))
 
 #define HVC_BCAST5(x)                       \
     v = __shfl(x, base + 0);                \
@@ -1014,7 +1008,6 @@ __device__ __forceinline__ GateK gate_k(const GateSlot& g)
     return GateK{A ? g.c : HR(0.0), g.type == 1 ? g.c : HR(0.0), g.type == 2 ? g.c : HR(0.0),
                  A ? -HR(1.0) : HR(1.0), -g.inv2_e, g.d, g.inv_e, g.c * g.e, A ? HR(0.5) * g.e : -HR(1.0)};
 }
-#ifdef HVC_FP32
 template <bool CAN_A>
 __device__ __forceinline__ real gate_rate_k(const GateK& g, real v)
 {
@@ -1032,7 +1025,6 @@ __device__ __forceinline__ real gate_rate_k(const GateK& g, real v)
     }
     return r;
 }
-#endif
 
 // derivatives of the lane's variable (kx) and, in lane 0, of w (kw) at stage
 // state (v, n1, m1, h1, w1); xo = the lane's own variable at the stage; w1 is
@@ -1043,7 +1035,6 @@ __device__ __forceinline__ void i_quad_rhs(Guard& bad, const IState& s, int role
                                            real e2, real e5, real& kx, real& kw)
 {
     HVC_FP_FAST
-#ifdef HVC_FP32
     // the same currents as one chain of multiply-adds: the two potassium
     // conductances share (v - E_K), the leak's reversal term is a constant
     // (the reference's closing "+ 100000 * 0 / A" only turns -0 into +0)
@@ -1072,16 +1063,6 @@ __device__ __forceinline__ void i_quad_rhs(Guard& bad, const IState& s, int role
             kg = __builtin_fmaf(-(a + b), xo, a);
         }
     }
-#else
-    real n4 = n1 * n1 * n1 * n1;
-    real m3 = m1 * m1 * m1;
-    real kV = -kI_gL * (v - kI_El) - kI_gNa * h1 * m3 * (v - kI_Ena) - kI_gKdr * n4 * (v - kI_Ek)
-                - kI_gKHT * w1 * (v - kI_Ek) - (s.Ge * e2) * v - (s.Gi * e5) * (v - kI_Ei) + 100000 * HR(0.0) / kI_A;
-    real a = gate_rate<EXACT>(bad, ga, v);
-    real b = gate_rate<EXACT>(bad, gb, v);
-    kw = role == 0 ? (a - w1) : HR(0.0);   // a = wInf in lane 0
-    real kg = a * (1 - xo) - b * xo;
-#endif
     kx = role == 0 ? kV : kg;
 }
 
@@ -1143,6 +1124,8 @@ __device__ __forceinline__ void i_dp8_quad(Guard& bad, IState& s, real& xlo, rea
 }
 #undef HVC_BCAST4
 
+#endif  // HVC_FP32
+
 // ---- HVC-I, DP8, eight lanes per neuron (octet) ----
 // Lanes q and 7 - q of a neuron's octet form a pair, exchanged by the DPP
 // half-row mirror: (1, 6) carry n and evaluate an / bn, (2, 5) m with am / bm,
@@ -1152,7 +1135,8 @@ __device__ __forceinline__ void i_dp8_quad(Guard& bad, IState& s, real& xlo, rea
 // owns V, lane 7 owns w and evaluates wInf.  A stage thus evaluates one rate
 // per lane (the quad two) and one stage combination (the quad two); lane 0's
 // membrane derivative gets n, m, h by quad broadcasts and w by the mirror.
-// Every value is the expression tree of HHI_buffer, as in i_dp8.
+// Every value is the expression tree of HHI_buffer, as in i_dp8.  (The FP64
+// form's stepper is in hvc_oct64.hip.h.)
 __constant__ GateSlot kIOctGates[8] = {
     {1, HR(0.0), HR(0.0), HR(10.0), HR(0.1), HVC_L2(10.0)},                 // V: no rate (unused)
     {0, HR(0.15), HR(15.0), HR(10.0), HR(0.1), HVC_L2(10.0)},               // an
@@ -1177,6 +1161,7 @@ __device__ __forceinline__ double oct_mirror(double x)
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+#ifdef HVC_FP32
 // derivative of the lane's variable at stage state (v, n1, m1, h1, w1); xo =
 // the lane's own variable at the stage; n1, m1, h1, w1 are needed in lane 0 only
 template <bool EXACT>
@@ -1184,7 +1169,6 @@ __device__ __forceinline__ real i_oct_rhs(Guard& bad, const IState& s, int q, co
                                           real m1, real h1, real w1, real xo, real e2, real e5)
 {
     HVC_FP_FAST
-#ifdef HVC_FP32
     const real n2 = n1 * n1;
     const real gk = __builtin_fmaf(kI_gKdr, n2 * n2, kI_gKHT * w1);
     real t = __builtin_fmaf(kI_gL, v, -(kI_gL * kI_El));
@@ -1205,16 +1189,6 @@ __device__ __forceinline__ real i_oct_rhs(Guard& bad, const IState& s, int q, co
     const real mr = oct_mirror(r);
     const real a = q < 4 ? r : mr, b = q < 4 ? mr : r;
     const real kg = __builtin_fmaf(-(a + b), xo, a);   // a (1 - x) - b x
-#else
-    real n4 = n1 * n1 * n1 * n1;
-    real m3 = m1 * m1 * m1;
-    real kV = -kI_gL * (v - kI_El) - kI_gNa * h1 * m3 * (v - kI_Ena) - kI_gKdr * n4 * (v - kI_Ek)
-                - kI_gKHT * w1 * (v - kI_Ek) - (s.Ge * e2) * v - (s.Gi * e5) * (v - kI_Ei) + 100000 * HR(0.0) / kI_A;
-    const real r = gate_rate<EXACT>(bad, g, v);
-    const real mr = oct_mirror(r);
-    const real a = q < 4 ? r : mr, b = q < 4 ? mr : r;
-    const real kg = a * (1 - xo) - b * xo;
-#endif
     const real kw = r - xo;   // lane 7: wInf - w
     return q == 0 ? kV : (q == 7 ? kw : kg);
 }
@@ -1246,7 +1220,6 @@ __device__ __forceinline__ void i_dp8_oct(Guard& bad, IState& s, real& xo, real&
     const real x0 = xo;
     real v = s.V, n1 = s.n, m1 = s.m, h1 = s.h, w1 = s.w;
     real x;
-#ifdef HVC_FP32
     // the step's decay factors of stages 3-13, read from LDS together before
     // the stages (each stage's read would otherwise wait on its own round trip)
     real e2r[11], e5r[11];
@@ -1259,20 +1232,11 @@ __device__ __forceinline__ void i_dp8_oct(Guard& bad, IState& s, real& xo, real&
     e5r[10] = row.e5[kOffDt];
 #define HVC_OE2(k, off) e2r[k]
 #define HVC_OE5(k, off) e5r[k]
-#else
-#define HVC_OE2(k, off) row.e2[off]
-#define HVC_OE5(k, off) row.e5[off]
-#endif
-// each stage derivative is noted once for all the tableau terms it enters
-#undef HVC_CKX
-#define HVC_CKX CKN
 #define HVC_OSTAGE(N, e2, e5, SX)                                                   \
     const real k_##N = i_oct_rhs<EXACT>(bad, s, q, g, v, n1, m1, h1, w1, x, e2, e5); \
-    bad.note_k(k_##N);                                                              \
     x = x0 + SX(k_);                                                                \
     HVC_BCAST8(x)
     const real k_1 = i_oct_rhs<EXACT>(bad, s, q, g, v, n1, m1, h1, w1, x0, HR(1.0), HR(1.0));
-    bad.note_k(k_1);
     x = x0 + HVC_DP8_S2(k_);
     HVC_BCAST8(x)
     HVC_OSTAGE(2, HVC_OE2(0, kOffDp2), HVC_OE5(0, kOffDp2), HVC_DP8_S3)
@@ -1287,7 +1251,6 @@ __device__ __forceinline__ void i_dp8_oct(Guard& bad, IState& s, real& xo, real&
     HVC_OSTAGE(11, HVC_OE2(9, kOffDp11), HVC_OE5(9, kOffDp11), HVC_DP8_S12)
 #undef HVC_OSTAGE
     const real k_12 = i_oct_rhs<EXACT>(bad, s, q, g, v, n1, m1, h1, w1, x, HVC_OE2(10, kOffDt), HVC_OE5(10, kOffDt));
-    bad.note_k(k_12);
 #undef HVC_OE2
 #undef HVC_OE5
     {
@@ -1302,9 +1265,8 @@ __device__ __forceinline__ void i_dp8_oct(Guard& bad, IState& s, real& xo, real&
     s.Ge = s.Ge * row_e2dt(row);
     s.Gi = s.Gi * row_e5dt(row);
 }
-#undef HVC_CKX
-#define HVC_CKX CK
 #undef HVC_BCAST8
+#endif  // HVC_FP32
 
 }  // namespace p32 / p64
 }  // namespace hvc
