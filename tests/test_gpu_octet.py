@@ -69,3 +69,29 @@ def test_large_network_takes_one_thread_per_neuron(model, n_ra):
                               erest=np.concatenate([small.erest, np.linspace(-90.0, -60.0, pad)]),
                               gca=np.concatenate([small.gca, np.linspace(0.0, 60.0, pad)]))
     _compare(net, 3.0, ra_model=model)
+
+
+@pytest.mark.parametrize("model,poisson", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("n,steps", [(1, 1), (8, 32), (9, 33), (33000, 3)])
+def test_trace_ra_sizes(model, poisson, n, steps):
+    """Chunk and block edges; the last size is beyond the octets."""
+    from oracle_lib import oracle, ra_inputs, run_ra_trace
+    from unsupervised_growth_amd.engine import Engine
+    inp = ra_inputs(n, steps, kick_step=min(2, steps - 1))
+    ref_state, ref_fired = run_ra_trace(oracle(), "ora", model, inp, poisson=poisson, seed=(7, 0), trial=2)
+    with Engine(ra_model=model, ra_poisson=poisson, seed=(7, 0)) as eng:
+        st, fi = eng.trace_ra(*inp, trial=2)
+    np.testing.assert_array_equal(fi, ref_fired)
+    np.testing.assert_array_equal(st, ref_state)
+
+
+@pytest.mark.parametrize("n,steps", [(1, 1), (8, 32), (9, 33), (20481, 14)])
+def test_trace_i_sizes(n, steps):
+    from oracle_lib import i_inputs, oracle, run_i_trace
+    from unsupervised_growth_amd.engine import Engine
+    inp = i_inputs(n, steps, exc_scale=0.3)
+    ref_state, ref_fired = run_i_trace(oracle(), "ora", 0, inp, first_trial=0, seed=(7, 0), trial=3)
+    with Engine(seed=(7, 0)) as eng:
+        st, fi = eng.trace_i(*inp, trial=3)
+    np.testing.assert_array_equal(fi, ref_fired)
+    np.testing.assert_array_equal(st, ref_state)

@@ -216,114 +216,6 @@ struct NoiseCursor {
     }
 };
 
-// ---------------------------------------------------------------------------
-// single-neuron traces
-// ---------------------------------------------------------------------------
-__global__ void k_trace_ra(NetDev nd, int n, int n_steps, uint32_t trial, const double* EL, const double* GCa,
-                           const double* kick, const double* exc_w, const double* inh_g, double* out, uint8_t* fired_out)
-{
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const DecayRow* rows = (const DecayRow*)nd.decay;
-    const RAUniform u = ra_uniform(nd);
-    // HH2_test::set_to_rest (HH2_test.cpp:196-205)
-    RAState s;
-    HVC_LOAD(s, Vs, -79.97619025) HVC_LOAD(s, Vd, -79.97268759) HVC_LOAD(s, n, 0.01101284)
-    HVC_LOAD(s, l, 0.0) HVC_LOAD(s, h, 0.9932845) HVC_LOAD(s, r, 0.00055429)
-    HVC_LOAD(s, c, 0.00000261762353) HVC_LOAD(s, Ca, 0.01689572)
-    s.Ge_s = 0; s.Gi_s = 0; s.Ge_d = 0; s.Gi_d = 0;
-    int fs = 0, fd = 0;
-    const real el = (real)EL[k], gca = (real)GCa[k];
-    PoissonStream ps{nd.seed_lo, nd.seed_hi, trial, kStreamRAPoisson, (uint32_t)k, 0u};
-    double nes = 0, nis = 0, ned = 0, nid = 0;
-    if (nd.ra_poisson) {
-        nes = 1000.0 * ps.spike_time(100.0);
-        nis = 1000.0 * ps.spike_time(100.0);
-        ned = 1000.0 * ps.spike_time(100.0);
-        nid = 1000.0 * ps.spike_time(100.0);
-    }
-    auto dump = [&](int row) {
-        double* o = out + ((size_t)row * n + k) * 12;
-        o[0] = HVC_WIDE(s, Vs); o[1] = HVC_WIDE(s, Vd); o[2] = HVC_WIDE(s, n); o[3] = HVC_WIDE(s, l);
-        o[4] = HVC_WIDE(s, h); o[5] = HVC_WIDE(s, r); o[6] = HVC_WIDE(s, c); o[7] = HVC_WIDE(s, Ca);
-        o[8] = s.Ge_s; o[9] = s.Gi_s; o[10] = s.Ge_d; o[11] = s.Gi_d;
-    };
-    dump(0);
-    for (int t = 1; t <= n_steps; ++t) {
-        size_t idx = (size_t)(t - 1) * n + k;
-        double kk = kick[idx];
-        if (kk != 0.0) s.Ge_d += kk;
-        int f = ra_state_check(s.Vs, s.Vd, fs, fd);
-        const DecayRow& row = rows[t];
-        if (nd.ra_model == 0) {
-            U4 o = philox4x32((uint32_t)t, (uint32_t)k, trial, kStreamRAWhite, nd.seed_lo, nd.seed_hi);
-            ra_step_debraband(s, el, gca, u, kPointDistribution[point_index(o.x)], kPointDistribution[point_index(o.y)],
-                         kPointDistribution[point_index(o.z)], kPointDistribution[point_index(o.w)],
-                         row.e5[kOffDt], row.e5[kOffHalf]);
-        } else {
-            if (nd.ra_poisson) {
-                double time = nd.clock[t - 1];
-                ra_noise_check(ps, time, nd.dt, s.Gi_s, 0.035, nis);
-                ra_noise_check(ps, time, nd.dt, s.Gi_d, 0.045, nid);
-                ra_noise_check(ps, time, nd.dt, s.Ge_s, 0.035, nes);
-                ra_noise_check(ps, time, nd.dt, s.Ge_d, 0.045, ned);
-            }
-            ra_step_runge4(s, el, gca, u, row.e5[kOffThird], row.e5[kOffTwoThird], row.e5[kOffDt]);
-        }
-        fired_out[idx] = (uint8_t)f;
-        double ig = inh_g[idx];
-        if (ig != 0.0) s.Gi_d += ig;
-        double ew = exc_w[idx];
-        if (ew != 0.0) s.Ge_d += ew / 10000.0;
-        dump(t);
-    }
-}
-
-__global__ void k_trace_i(NetDev nd, int n, int n_steps, int first_trial, uint32_t trial, const double* exc_g,
-                          const double* inh_g, double* out, uint8_t* fired_out)
-{
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const DecayRow* rows = (const DecayRow*)nd.decay;
-    // HHI_buffer::set_to_rest (HHI_buffer.cpp:181-185)
-    IState s;
-    HVC_LOAD(s, V, -66.0) HVC_LOAD(s, n, 0.125) HVC_LOAD(s, m, 0.0) HVC_LOAD(s, h, 0.99) HVC_LOAD(s, w, 0.0)
-    s.Ge = 0; s.Gi = 0;
-    int flag = 0;
-    PoissonStream ps{nd.seed_lo, nd.seed_hi, trial, kStreamIPoisson, (uint32_t)k, 0u};
-    double ne = 0, ni = 0;
-    if (nd.i_poisson) {
-        double init_dt = first_trial ? 0.0 : nd.dt;
-        ne = i_init_noise(ps, init_dt);
-        ni = i_init_noise(ps, init_dt);
-    }
-    auto dump = [&](int row) {
-        double* o = out + ((size_t)row * n + k) * 7;
-        o[0] = HVC_WIDE(s, V); o[1] = HVC_WIDE(s, n); o[2] = HVC_WIDE(s, m); o[3] = HVC_WIDE(s, h);
-        o[4] = HVC_WIDE(s, w); o[5] = s.Ge; o[6] = s.Gi;
-    };
-    dump(0);
-    for (int t = 1; t <= n_steps; ++t) {
-        size_t idx = (size_t)(t - 1) * n + k;
-        int f = i_state_check(s.V, flag);
-        if (nd.i_poisson) {
-            double time = nd.clock[t - 1];
-            i_noise_check(ps, time, nd.dt, s.Ge, ne);
-            i_noise_check(ps, time, nd.dt, s.Gi, ni);
-        }
-        if (nd.i_model == 0)
-            i_step<0>(s, nd.dt, rows[t]);
-        else
-            i_step<1>(s, (real)nd.dt, rows[t]);
-        fired_out[idx] = (uint8_t)f;
-        double ig = inh_g[idx];
-        if (ig != 0.0) s.Gi += ig;
-        double eg = exc_g[idx];
-        if (eg != 0.0) s.Ge += eg;
-        dump(t);
-    }
-}
-
 // append (neuron, step) to a log with one atomic per wave
 __device__ __forceinline__ void wave_append(int2* log, int* cnt, int cap, bool pred, int neuron, int step,
                                             unsigned int* err)
@@ -1050,6 +942,301 @@ __global__ __launch_bounds__(256) void k_integrate(NetDev nd, int t0, int t1, in
 #endif
 }
 
+// ---------------------------------------------------------------------------
+// single-neuron traces.  A trace is one serial chain of steps per neuron, so
+// what a step waits on is what it costs: the decay rows and the clock of
+// kTraceChunk steps are staged in LDS, and a step's inputs are loaded a step
+// ahead (one thread per neuron) or with the chunk (octets).  One wave per block,
+// said so to the compiler (without launch bounds the kernels were held to 128
+// registers and spilled 640-780 bytes).  Whole calls, before and now: 16
+// HVC-RA neurons x 500 steps FP64 5.6 -> 1.5 ms, 330 HVC-I x 1 250 FP64 33 ->
+// 6.8 ms (both octets), 2 000 HVC-RA x 1 500 FP32 (one thread) 3.5 -> 2.2 ms.
+// ---------------------------------------------------------------------------
+constexpr int kTraceChunk = 32;
+constexpr size_t kTraceLds = kTraceChunk * sizeof(WinRow) + (kTraceChunk + 1) * sizeof(double);
+
+// the chunk's tables for the steps t0 .. t1, staged by the block
+__device__ __forceinline__ Win trace_window(const NetDev& nd, double* lds, int t0, int t1)
+{
+    const int nsteps = t1 - t0 + 1;
+    const Win win{(const WinRow*)lds, (const double*)((const WinRow*)lds + nsteps), t0, lds, nsteps};
+    __syncthreads();   // the previous chunk's tables are done with
+    win.stage(nd);
+    return win;
+}
+
+// the four Poisson channels of an HVC-RA trace (HH2_buffer's initial draws and checks)
+struct RATraceNoise {
+    PoissonStream ps;
+    double nes, nis, ned, nid;
+    __device__ __forceinline__ RATraceNoise(const NetDev& nd, uint32_t trial, int k)
+        : ps{nd.seed_lo, nd.seed_hi, trial, kStreamRAPoisson, (uint32_t)k, 0u}, nes(0), nis(0), ned(0), nid(0)
+    {
+        if (nd.ra_poisson) {
+            nes = 1000.0 * ps.spike_time(100.0);
+            nis = 1000.0 * ps.spike_time(100.0);
+            ned = 1000.0 * ps.spike_time(100.0);
+            nid = 1000.0 * ps.spike_time(100.0);
+        }
+    }
+    __device__ __forceinline__ void check(double time, double dt, real& Ge_s, real& Gi_s, real& Ge_d, real& Gi_d)
+    {
+        ra_noise_check(ps, time, dt, Gi_s, 0.035, nis);
+        ra_noise_check(ps, time, dt, Gi_d, 0.045, nid);
+        ra_noise_check(ps, time, dt, Ge_s, 0.035, nes);
+        ra_noise_check(ps, time, dt, Ge_d, 0.045, ned);
+    }
+};
+
+__global__ __launch_bounds__(64) void k_trace_ra(NetDev nd, int n, int n_steps, uint32_t trial, const double* EL,
+                                                 const double* GCa, const double* kick, const double* exc_w,
+                                                 const double* inh_g, double* out, uint8_t* fired_out)
+{
+    extern __shared__ double trace_lds[];
+    const int k0 = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = k0 < n;
+    const int k = live ? k0 : n - 1;
+    const RAUniform u = ra_uniform(nd);
+    // HH2_test::set_to_rest (HH2_test.cpp:196-205)
+    RAState s;
+    HVC_LOAD(s, Vs, -79.97619025) HVC_LOAD(s, Vd, -79.97268759) HVC_LOAD(s, n, 0.01101284)
+    HVC_LOAD(s, l, 0.0) HVC_LOAD(s, h, 0.9932845) HVC_LOAD(s, r, 0.00055429)
+    HVC_LOAD(s, c, 0.00000261762353) HVC_LOAD(s, Ca, 0.01689572)
+    s.Ge_s = 0; s.Gi_s = 0; s.Ge_d = 0; s.Gi_d = 0;
+    int fs = 0, fd = 0;
+    const real el = (real)EL[k], gca = (real)GCa[k];
+    RATraceNoise pn(nd, trial, k);
+    auto dump = [&](int row) {
+        if (!live) return;
+        double* o = out + ((size_t)row * n + k) * 12;
+        o[0] = HVC_WIDE(s, Vs); o[1] = HVC_WIDE(s, Vd); o[2] = HVC_WIDE(s, n); o[3] = HVC_WIDE(s, l);
+        o[4] = HVC_WIDE(s, h); o[5] = HVC_WIDE(s, r); o[6] = HVC_WIDE(s, c); o[7] = HVC_WIDE(s, Ca);
+        o[8] = s.Ge_s; o[9] = s.Gi_s; o[10] = s.Ge_d; o[11] = s.Gi_d;
+    };
+    dump(0);
+    double kk = kick[k], ig = inh_g[k], ew = exc_w[k];   // the next step's inputs
+    for (int t0 = 1; t0 <= n_steps; t0 += kTraceChunk) {
+        const int t1 = min(t0 + kTraceChunk - 1, n_steps);
+        const Win win = trace_window(nd, trace_lds, t0, t1);
+        for (int t = t0; t <= t1; ++t) {
+            const size_t idx = (size_t)(t - 1) * n + k, nxt = (size_t)min(t, n_steps - 1) * n + k;
+            const double kn = kick[nxt], in = inh_g[nxt], en = exc_w[nxt];
+            if (kk != 0.0) s.Ge_d += kk;
+            int f = ra_state_check(s.Vs, s.Vd, fs, fd);
+            const WinRow& row = win.row(t);
+            if (nd.ra_model == 0) {
+                U4 o = philox4x32((uint32_t)t, (uint32_t)k, trial, kStreamRAWhite, nd.seed_lo, nd.seed_hi);
+                ra_step_debraband(s, el, gca, u, kPointDistribution[point_index(o.x)],
+                                  kPointDistribution[point_index(o.y)], kPointDistribution[point_index(o.z)],
+                                  kPointDistribution[point_index(o.w)], row.e5[kOffDt], row.e5[kOffHalf]);
+            } else {
+                if (nd.ra_poisson) pn.check(win.clk(t - 1), nd.dt, s.Ge_s, s.Gi_s, s.Ge_d, s.Gi_d);
+                ra_step_runge4(s, el, gca, u, row.e5[kOffThird], row.e5[kOffTwoThird], row.e5[kOffDt]);
+            }
+            if (live) fired_out[idx] = (uint8_t)f;
+            if (ig != 0.0) s.Gi_d += ig;
+            if (ew != 0.0) s.Ge_d += ew / 10000.0;
+            dump(t);
+            kk = kn;
+            ig = in;
+            ew = en;
+        }
+    }
+}
+
+__global__ __launch_bounds__(64) void k_trace_i(NetDev nd, int n, int n_steps, int first_trial, uint32_t trial,
+                                                const double* exc_g, const double* inh_g, double* out,
+                                                uint8_t* fired_out)
+{
+    extern __shared__ double trace_lds[];
+    const int k0 = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = k0 < n;
+    const int k = live ? k0 : n - 1;
+    // HHI_buffer::set_to_rest (HHI_buffer.cpp:181-185)
+    IState s;
+    HVC_LOAD(s, V, -66.0) HVC_LOAD(s, n, 0.125) HVC_LOAD(s, m, 0.0) HVC_LOAD(s, h, 0.99) HVC_LOAD(s, w, 0.0)
+    s.Ge = 0; s.Gi = 0;
+    int flag = 0;
+    PoissonStream ps{nd.seed_lo, nd.seed_hi, trial, kStreamIPoisson, (uint32_t)k, 0u};
+    double ne = 0, ni = 0;
+    if (nd.i_poisson) {
+        double init_dt = first_trial ? 0.0 : nd.dt;
+        ne = i_init_noise(ps, init_dt);
+        ni = i_init_noise(ps, init_dt);
+    }
+    auto dump = [&](int row) {
+        if (!live) return;
+        double* o = out + ((size_t)row * n + k) * 7;
+        o[0] = HVC_WIDE(s, V); o[1] = HVC_WIDE(s, n); o[2] = HVC_WIDE(s, m); o[3] = HVC_WIDE(s, h);
+        o[4] = HVC_WIDE(s, w); o[5] = s.Ge; o[6] = s.Gi;
+    };
+    dump(0);
+    double ig = inh_g[k], eg = exc_g[k];   // the next step's inputs
+    for (int t0 = 1; t0 <= n_steps; t0 += kTraceChunk) {
+        const int t1 = min(t0 + kTraceChunk - 1, n_steps);
+        const Win win = trace_window(nd, trace_lds, t0, t1);
+        for (int t = t0; t <= t1; ++t) {
+            const size_t idx = (size_t)(t - 1) * n + k, nxt = (size_t)min(t, n_steps - 1) * n + k;
+            const double in = inh_g[nxt], en = exc_g[nxt];
+            int f = i_state_check(s.V, flag);
+            if (nd.i_poisson) {
+                const double time = win.clk(t - 1);
+                i_noise_check(ps, time, nd.dt, s.Ge, ne);
+                i_noise_check(ps, time, nd.dt, s.Gi, ni);
+            }
+            if (nd.i_model == 0)
+                i_step<0>(s, nd.dt, win.row(t));
+            else
+                i_step<1>(s, (real)nd.dt, win.row(t));
+            if (live) fired_out[idx] = (uint8_t)f;
+            if (ig != 0.0) s.Gi += ig;
+            if (eg != 0.0) s.Ge += eg;
+            dump(t);
+            ig = in;
+            eg = en;
+        }
+    }
+}
+
+#ifndef HVC_FP32
+// Traces on octets: eight neurons per block.  Lane q stores its own variable;
+// lane 0 (HVC-RA: lanes 0 and 5) also stores the conductances.
+__device__ __forceinline__ void trace_inputs(double* lds, const double* src, int k0, int n, int t0, int t1)
+{
+    for (int r = threadIdx.x; r < 8 * (t1 - t0 + 1); r += blockDim.x)
+        lds[r] = src[(size_t)(t0 - 1 + (r >> 3)) * n + min(k0 + (r & 7), n - 1)];
+}
+
+template <int MODEL>
+__global__ __launch_bounds__(64) void k_trace_ra_oct(NetDev nd, int n, int n_steps, uint32_t trial, const double* EL,
+                                                     const double* GCa, const double* kick, const double* exc_w,
+                                                     const double* inh_g, double* out, uint8_t* fired_out)
+{
+    extern __shared__ double trace_lds[];
+    __shared__ ExpPair exp_tab[64];
+    __shared__ RANoise noise_rows[MODEL == 0 ? kNoiseRows : 1];
+    __shared__ uint8_t noise_at[8 * 2 * kTraceChunk];
+    __shared__ double in_kick[8 * kTraceChunk], in_exc[8 * kTraceChunk], in_inh[8 * kTraceChunk];
+    const int lane = threadIdx.x, q = lane & 7, g = lane >> 3;
+    const bool live = (int)blockIdx.x * 8 + g < n;
+    const int k = live ? blockIdx.x * 8 + g : n - 1;
+    stage_exp_table(exp_tab);
+    if constexpr (MODEL == 0) stage_noise_rows(noise_rows, nd.sq_sig_s, nd.sq_sig_d);
+    const RAOctLane L = ra_oct_lane<MODEL>(q, EL[k], GCa[k], nd.mu_term_s, nd.mu_term_d, exp_tab);
+    // HH2_test::set_to_rest (HH2_test.cpp:196-205), by state variable
+    const int var = ra_oct_var(q);
+    double x = var == 0 ? -79.97619025 : var == 1 ? -79.97268759 : var == 2 ? 0.01101284 : var == 3 ? 0.0
+             : var == 4 ? 0.9932845 : var == 5 ? 0.00055429 : var == 6 ? 0.00000261762353 : 0.01689572;
+    double GA = 0, GB = 0;   // Gi_s, Ge_s in lane 0; Ge_d, Gi_d in lane 5
+    int flag = 0;
+    RATraceNoise pn(nd, trial, k);
+    const NoiseId sid{nd.seed_lo, nd.seed_hi, trial, (uint32_t)k};
+    auto dump = [&](int row) {
+        if (!live) return;
+        double* o = out + ((size_t)row * n + k) * 12;
+        o[var] = MODEL == 1 && q == 3 ? 0.0 : x;
+        if (q == 0) { o[8] = GB; o[9] = GA; }
+        if (q == 5) { o[10] = GA; o[11] = GB; }
+    };
+    dump(0);
+    for (int t0 = 1; t0 <= n_steps; t0 += kTraceChunk) {
+        const int t1 = min(t0 + kTraceChunk - 1, n_steps);
+        __syncthreads();
+        trace_inputs(in_kick, kick, blockIdx.x * 8, n, t0, t1);
+        trace_inputs(in_exc, exc_w, blockIdx.x * 8, n, t0, t1);
+        trace_inputs(in_inh, inh_g, blockIdx.x * 8, n, t0, t1);
+        uint8_t* at = noise_at + g * 2 * kTraceChunk;
+        if constexpr (MODEL == 0) noise_window(at, q, sid, t0, t1 - t0 + 1);
+        const Win win = trace_window(nd, trace_lds, t0, t1);
+        for (int t = t0; t <= t1; ++t) {
+            const int r = (t - t0) * 8 + g;
+            const double kk = in_kick[r], ig = in_inh[r], ew = in_exc[r];
+            if (q == 5 && kk != 0.0) GA += kk;
+            const int f = ra_oct_check(q, x, flag);
+            RANoise nz{};
+            if constexpr (MODEL == 0) {
+                const int j = 2 * (t - t0);
+                nz = noise_rows[q == 0 ? at[j] : (q == 5 ? at[j + 1] : kNoiseRows - 1)];
+            } else if (nd.ra_poisson) {
+                double other = 0.0;
+                const bool dend = q == 5;
+                double ges = dend ? other : GB, gis = dend ? other : GA, ged = dend ? GA : other, gid = dend ? GB : other;
+                pn.check(win.clk(t - 1), nd.dt, ges, gis, ged, gid);
+                GA = dend ? ged : gis;
+                GB = dend ? gid : ges;
+            }
+            ra_oct_step<MODEL>(L, x, GA, GB, nd.dt, nz, win.row(t));
+            const uint64_t fired = __ballot(f != 0) >> (lane & ~7);
+            if (live && q == 0)
+                fired_out[(size_t)(t - 1) * n + k] = (uint8_t)((fired & 1u) | ((fired >> 4) & 2u));
+            if (q == 5) {
+                if (ig != 0.0) GB += ig;
+                if (ew != 0.0) GA += ew / 10000.0;
+            }
+            dump(t);
+        }
+    }
+}
+
+__global__ __launch_bounds__(64) void k_trace_i_oct(NetDev nd, int n, int n_steps, int first_trial, uint32_t trial,
+                                                    const double* exc_g, const double* inh_g, double* out,
+                                                    uint8_t* fired_out)
+{
+    extern __shared__ double trace_lds[];
+    __shared__ ExpPair exp_tab[64];
+    __shared__ double in_exc[8 * kTraceChunk], in_inh[8 * kTraceChunk];
+    const int lane = threadIdx.x, q = lane & 7, g = lane >> 3;
+    const bool live = (int)blockIdx.x * 8 + g < n;
+    const int k = live ? blockIdx.x * 8 + g : n - 1;
+    stage_exp_table(exp_tab);
+    const IOctLane L = i_oct_lane(q, exp_tab);
+    // HHI_buffer::set_to_rest (HHI_buffer.cpp:181-185), by state variable; the
+    // mirror lanes 4-6 carry 1 - x
+    const int var = i_oct_var(q);
+    double x = var == 0 ? -66.0 : var == 1 ? 0.125 : var == 2 ? 0.0 : var == 3 ? 0.99 : 0.0;
+    if (q > 3 && q < 7) x = 1 - x;
+    double Ge = 0, Gi = 0;
+    int flag = 0;
+    PoissonStream ps{nd.seed_lo, nd.seed_hi, trial, kStreamIPoisson, (uint32_t)k, 0u};
+    double ne = 0, ni = 0;
+    if (nd.i_poisson) {
+        double init_dt = first_trial ? 0.0 : nd.dt;
+        ne = i_init_noise(ps, init_dt);
+        ni = i_init_noise(ps, init_dt);
+    }
+    auto dump = [&](int row) {
+        double* o = out + ((size_t)row * n + k) * 7;
+        if (live && (q < 4 || q == 7)) o[var] = x;
+        if (live && q == 0) { o[5] = Ge; o[6] = Gi; }
+    };
+    dump(0);
+    Dp8Consts C;
+    dp8_pin(C);
+    for (int t0 = 1; t0 <= n_steps; t0 += kTraceChunk) {
+        const int t1 = min(t0 + kTraceChunk - 1, n_steps);
+        __syncthreads();
+        trace_inputs(in_exc, exc_g, blockIdx.x * 8, n, t0, t1);
+        trace_inputs(in_inh, inh_g, blockIdx.x * 8, n, t0, t1);
+        const Win win = trace_window(nd, trace_lds, t0, t1);
+        for (int t = t0; t <= t1; ++t) {
+            const int r = (t - t0) * 8 + g;
+            const double ig = in_inh[r], eg = in_exc[r];
+            const int f = i_state_check(x, flag);   // of V in lane 0
+            if (nd.i_poisson) {
+                const double time = win.clk(t - 1);
+                i_noise_check(ps, time, nd.dt, Ge, ne);
+                i_noise_check(ps, time, nd.dt, Gi, ni);
+            }
+            i_oct_step(L, C, x, Ge, Gi, nd.dt, win.row(t));
+            if (live && q == 0) fired_out[(size_t)(t - 1) * n + k] = (uint8_t)f;
+            if (ig != 0.0) Gi += ig;
+            if (eg != 0.0) Ge += eg;
+            dump(t);
+        }
+    }
+}
+#endif
+
 // LDS bytes of k_integrate for a window of n steps
 static inline size_t win_bytes(int n) { return (size_t)n * sizeof(WinRow) + (size_t)(n + 1) * sizeof(double); }
 
@@ -1064,6 +1251,10 @@ static inline size_t win_bytes(int n) { return (size_t)n * sizeof(WinRow) + (siz
 // 20 000 neurons, 106 / 116 at 30 000, 134 / 117 at 40 000; RK4 76 / 82 at
 // 20 000, 99 / 99 at 30 000, 126 / 99 at 40 000.
 constexpr int kRAOctMaxNeurons[2] = {32768, 16384};   // by ra_model
+// HVC-I neurons up to which a trace takes octets (a trace has no launch shape):
+// beside one-thread HVC-RA waves k_integrate takes 149 us per window with
+// octets, 204 with one thread at 16 500 HVC-I neurons, 224 / 206 at 24 750
+constexpr int kIOctMaxTraces = 20480;
 #endif
 
 #ifdef HVC_FP32
@@ -1076,13 +1267,32 @@ void HVC_LAUNCHER(launch_trace_ra)(hipStream_t st, const NetDev& nd, int n, int 
                      const double* GCa, const double* kick, const double* exc_w, const double* inh_g, double* out,
                      uint8_t* fired)
 {
-    k_trace_ra<<<blocks_for(n, 64), 64, 0, st>>>(nd, n, n_steps, trial, EL, GCa, kick, exc_w, inh_g, out, fired);
+#ifndef HVC_FP32
+    if (n <= kRAOctMaxNeurons[nd.ra_model == 1]) {
+        if (nd.ra_model == 0)
+            k_trace_ra_oct<0><<<blocks_for(n, 8), 64, kTraceLds, st>>>(nd, n, n_steps, trial, EL, GCa, kick, exc_w,
+                                                                       inh_g, out, fired);
+        else
+            k_trace_ra_oct<1><<<blocks_for(n, 8), 64, kTraceLds, st>>>(nd, n, n_steps, trial, EL, GCa, kick, exc_w,
+                                                                       inh_g, out, fired);
+        return;
+    }
+#endif
+    k_trace_ra<<<blocks_for(n, 64), 64, kTraceLds, st>>>(nd, n, n_steps, trial, EL, GCa, kick, exc_w, inh_g, out,
+                                                         fired);
 }
 
 void HVC_LAUNCHER(launch_trace_i)(hipStream_t st, const NetDev& nd, int n, int n_steps, int first_trial, uint32_t trial,
                     const double* exc_g, const double* inh_g, double* out, uint8_t* fired)
 {
-    k_trace_i<<<blocks_for(n, 64), 64, 0, st>>>(nd, n, n_steps, first_trial, trial, exc_g, inh_g, out, fired);
+#ifndef HVC_FP32
+    if (nd.i_model == 0 && n <= kIOctMaxTraces) {
+        k_trace_i_oct<<<blocks_for(n, 8), 64, kTraceLds, st>>>(nd, n, n_steps, first_trial, trial, exc_g, inh_g, out,
+                                                               fired);
+        return;
+    }
+#endif
+    k_trace_i<<<blocks_for(n, 64), 64, kTraceLds, st>>>(nd, n, n_steps, first_trial, trial, exc_g, inh_g, out, fired);
 }
 
 void HVC_LAUNCHER(launch_integrate)(hipStream_t st, const NetDev& nd, int t0, int t1, const Tuning& tu,
