@@ -95,3 +95,32 @@ def test_trace_i_sizes(n, steps):
         st, fi = eng.trace_i(*inp, trial=3)
     np.testing.assert_array_equal(fi, ref_fired)
     np.testing.assert_array_equal(st, ref_state)
+
+
+@pytest.mark.parametrize("model,ra_lanes", [(1, 0), (1, 1), (0, 0)])
+def test_fp32_one_thread_shape_on_octets(model, ra_lanes):
+    """A small FP32 network whose shape asks for one thread per HVC-I neuron
+    equals the same network in a batch too large for octets (spikes: the rates
+    pass their series near v = -15 and v = -22)."""
+    from unsupervised_growth_amd.engine import Engine
+    from unsupervised_growth_amd.network import random_network
+    net = random_network(40, 37, n_train=8, p_ra2i=0.5, p_i2ra=0.3, gei_max=2.0, seed=3)
+    i = 10241
+    z, f = np.zeros(2, np.int32), np.zeros(0, np.int32)
+    e = np.zeros(0)
+    idle = dataclasses.replace(net, n_ra=1, n_i=i, ra2i_ptr=z, ra2i_tgt=f, ra2i_w=e, ra2i_d=e,
+                               i2ra_ptr=np.zeros(i + 1, np.int32), i2ra_tgt=f, i2ra_w=e, i2ra_d=e, rr_ptr=z, rr_tgt=f,
+                               rr_d=e, rr_w=e, act_cnt=z[:1], act_ids=f, sup_cnt=z[:1], sup_ids=f, remodeled=z[:1],
+                               erest=net.erest[:1], gca=net.gca[:1], train_ids=f, spread=e)
+    kw = dict(precision=1, trial_ms=100.0, ra_model=model)
+    tr = dict(mode=0, trial_index=0, first_trial=True, mean_injection_time=10.0)
+    with Engine(seed=(5, 0), **kw) as a, Engine(**kw) as b:
+        a.upload(net)
+        b.upload_batch([net, idle], [(5, 0), (6, 0)])
+        for x in (a, b):
+            x.set_tuning(i_lanes=0, ra_lanes=ra_lanes)
+        ra, rb = a.run_trial(**tr), b.run_batch([tr, tr])[0]
+    assert sum(map(len, ra.interneuron)) > 0
+    for kind in ("soma", "dend", "interneuron"):
+        for x, y in zip(getattr(ra, kind), getattr(rb, kind)):
+            np.testing.assert_array_equal(x, y)

@@ -120,6 +120,14 @@ __device__ __forceinline__ void i_step_oct(IState& s, real& xo, real& xlo, int q
     Guard bad;
     i_dp8_oct<false>(bad, s, xo, xlo, q, g, dt, row);
 }
+template <class Row>
+__device__ __forceinline__ void i_step_oct(IState& s, real& xo, real& xlo, int q, const IOctShared& g, real dt,
+                                           const Row& row)
+{
+    i_dp8_shared(s, xo, xlo, q, g, dt, row);
+}
+__device__ __forceinline__ void i_oct_gate(GateSlot& g, int q) { g = kIOctGates[q]; }
+__device__ __forceinline__ void i_oct_gate(IOctShared& g, int q) { g = IOctShared(q); }
 #endif
 #undef HVC_GUARDED_STEP
 
@@ -648,7 +656,9 @@ __device__ void integrate_i_quad(const NetDev& nd, const Win& win, int wave, int
 constexpr int kINeuronsPerOctWave = 8;       // eight lanes per HVC-I neuron
 
 #ifdef HVC_FP32
-// HVC-I, eight lanes per neuron (DP8 form); one wave holds 8 neurons
+// HVC-I, eight lanes per neuron (DP8 form); one wave holds 8 neurons.  Gate:
+// the arithmetic of the gates (GateSlot: the octet's own, IOctShared: the one-thread stepper's)
+template <class Gate>
 __device__ void integrate_i_oct(const NetDev& nd, const Win& win, int wave, int t0, int t1)
 {
     const int lane = __lane_id();
@@ -656,7 +666,8 @@ __device__ void integrate_i_oct(const NetDev& nd, const Win& win, int wave, int 
     const int i = wave * kINeuronsPerOctWave + (lane >> 3);
     const bool live = i < nd.n_i && (!nd.net_live || nd.net_live[nd.i_net[i]]);
     const int ii = live ? i : 0;
-    const GateSlot g = kIOctGates[q];
+    Gate g;
+    i_oct_gate(g, q);
     // the lane's own variable: V (lane 0), n (1, 6), m (2, 5), h (3, 4), w (7)
     const int var = q == 0 ? 0 : (q == 1 || q == 6 ? 1 : (q == 2 || q == 5 ? 2 : (q == 7 ? 4 : 3)));
     IState s;
@@ -887,7 +898,8 @@ __device__ void integrate_ra_oct(const NetDev& nd, const Win& win, const OctLds&
 // of LANES; any blocks after them run the previous window's sync-point STDP
 // (one row per thread, sa).
 // LANES: HVC-I bit 0 = five lanes, bit 2 = four lanes, bit 3 = eight lanes per
-// neuron, none = one thread; HVC-RA bit 1 = four lanes (FP32 form) or eight
+// neuron, bit 4 = eight lanes with the one-thread arithmetic (FP32 form), none
+// = one thread; HVC-RA bit 1 = four lanes (FP32 form) or eight
 // (FP64 form), else one thread.  (The layouts are template parameters: a
 // kernel holds the register allocation of one layout only.  The FP64 form has
 // the octets and one thread.)
@@ -909,8 +921,10 @@ __global__ __launch_bounds__(256) void k_integrate(NetDev nd, int t0, int t1, in
     const int rwave = (blockIdx.x - iblocks) * (blockDim.x >> 6) + (threadIdx.x >> 6);
 #ifdef HVC_FP32
     if ((int)blockIdx.x < iblocks) {
-        if constexpr ((LANES & 8) != 0)
-            integrate_i_oct(nd, win, iwave, t0, t1);
+        if constexpr ((LANES & 16) != 0)
+            integrate_i_oct<IOctShared>(nd, win, iwave, t0, t1);
+        else if constexpr ((LANES & 8) != 0)
+            integrate_i_oct<GateSlot>(nd, win, iwave, t0, t1);
         else if constexpr ((LANES & 4) != 0)
             integrate_i_quad(nd, win, iwave, t0, t1);
         else if constexpr ((LANES & 1) != 0)
@@ -1242,7 +1256,14 @@ static inline size_t win_bytes(int n) { return (size_t)n * sizeof(WinRow) + (siz
 
 }  // namespace p32 / p64
 
-#ifndef HVC_FP32
+#ifdef HVC_FP32
+// HVC-I neurons per context up to which "one thread per neuron" runs on eight
+// lanes with the one-thread stepper's arithmetic.  k_integrate per window
+// (HVC-RA one thread per neuron beside it, 3.6 times as many; the launch
+// included), octets / one thread, us: 25 / 41 at 2 750 HVC-I neurons, 35 / 42
+// at 8 745, 41 / 42 at 12 400, 43 / 43 at 16 000.
+constexpr int kIOctSharedMaxNeurons = 10240;
+#else
 // HVC-RA neurons per context up to which a window takes octets without being
 // asked.  An octet's wave is short (640 instructions per Debraband step, the
 // one-thread wave 5 600 before the two-operation quotients, 4 700 with them)
@@ -1302,12 +1323,14 @@ void HVC_LAUNCHER(launch_integrate)(hipStream_t st, const NetDev& nd, int t0, in
     const int wpb = bs / 64;
 #ifdef HVC_FP32
     // HVC-I layout (DP8 only): 0 one thread, 1 five lanes, 2 four lanes, 3 eight lanes per neuron
-    const int i_layout = nd.i_model == 0 ? tu.i_lanes : 0;
+    // (or 4: the one-thread form's arithmetic on eight lanes, while the HVC-I
+    // waves of that layout still find SIMDs to run on)
+    const int i_layout = nd.i_model != 0 ? 0 : (tu.i_lanes == 0 && nd.n_i <= kIOctSharedMaxNeurons ? 4 : tu.i_lanes);
     const int ra_lanes = (nd.ra_model == 1 && tu.ra_lanes) ? 1 : 0;
     const int ra_per_block = ra_lanes ? wpb * kRANeuronsPerWave : bs;
     const int i_per_block = i_layout == 1 ? wpb * kINeuronsPerWave
                             : (i_layout == 2 ? wpb * kINeuronsPerQuadWave
-                                             : (i_layout == 3 ? wpb * kINeuronsPerOctWave : bs));
+                                             : (i_layout >= 3 ? wpb * kINeuronsPerOctWave : bs));
 #else
     // the FP64 layouts give the same bits, so every HVC-I layout with several
     // lanes is the octet (45 us per window at 2 000 + 550 neurons; the four-lane
@@ -1327,18 +1350,21 @@ void HVC_LAUNCHER(launch_integrate)(hipStream_t st, const NetDev& nd, int t0, in
 #ifdef HVC_FP32
     if (nd.ra_model == 0) {
         if (nd.i_model == 1) HVC_K(0, 1, 0);
+        else if (i_layout == 4) HVC_K(0, 0, 16);
         else if (i_layout == 3) HVC_K(0, 0, 8);
         else if (i_layout == 2) HVC_K(0, 0, 4);
         else if (i_layout == 1) HVC_K(0, 0, 1);
         else HVC_K(0, 0, 0);
     } else if (ra_lanes) {
         if (nd.i_model == 1) HVC_K(1, 1, 2);
+        else if (i_layout == 4) HVC_K(1, 0, 18);
         else if (i_layout == 3) HVC_K(1, 0, 10);
         else if (i_layout == 2) HVC_K(1, 0, 6);
         else if (i_layout == 1) HVC_K(1, 0, 3);
         else HVC_K(1, 0, 2);
     } else {
         if (nd.i_model == 1) HVC_K(1, 1, 0);
+        else if (i_layout == 4) HVC_K(1, 0, 16);
         else if (i_layout == 3) HVC_K(1, 0, 8);
         else if (i_layout == 2) HVC_K(1, 0, 4);
         else if (i_layout == 1) HVC_K(1, 0, 1);

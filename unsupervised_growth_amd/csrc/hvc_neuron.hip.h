@@ -1130,9 +1130,8 @@ __device__ __forceinline__ void i_dp8_quad(Guard& bad, IState& s, real& xlo, rea
 // Lanes q and 7 - q of a neuron's octet form a pair, exchanged by the DPP
 // half-row mirror: (1, 6) carry n and evaluate an / bn, (2, 5) m with am / bm,
 // (3, 4) h with ah / bh.  Each lane of a pair evaluates one of its variable's
-// two rates, takes the other from its partner and advances the variable with
-// the same operations on the same values, so both hold the same bits.  Lane 0
-// owns V, lane 7 owns w and evaluates wInf.  A stage thus evaluates one rate
+// two rates; the lower lane owns the variable and takes the other rate from its
+// partner.  Lane 0 owns V, lane 7 owns w and evaluates wInf.  A stage thus evaluates one rate
 // per lane (the quad two) and one stage combination (the quad two); lane 0's
 // membrane derivative gets n, m, h by quad broadcasts and w by the mirror.
 // Every value is the expression tree of HHI_buffer, as in i_dp8.  (The FP64
@@ -1186,23 +1185,29 @@ __device__ __forceinline__ real i_oct_rhs(Guard& bad, const IState& s, int q, co
         const real sr = gk1.ce * xexpm1_series(vd * gk1.ie);
         if (near) r = sr;
     }
+    // n, m, h live in lanes 1-3 (their mirror lanes only evaluate rates)
     const real mr = oct_mirror(r);
-    const real a = q < 4 ? r : mr, b = q < 4 ? mr : r;
-    const real kg = __builtin_fmaf(-(a + b), xo, a);   // a (1 - x) - b x
+    const real kg = __builtin_fmaf(-(r + mr), xo, r);   // a (1 - x) - b x
     const real kw = r - xo;   // lane 7: wInf - w
     return q == 0 ? kV : (q == 7 ? kw : kg);
 }
 
+// lane LO of the quad of x in an octet's lanes 0-3, lane HI of the quad of y in
+// its lanes 4-7
+template <int LO, int HI>
+__device__ __forceinline__ float half_bcast(float x, float y)
+{
+    const int a = __builtin_amdgcn_mov_dpp(__float_as_int(x), LO * 0x55, 0xF, 0xF, true);
+    return __int_as_float(__builtin_amdgcn_update_dpp(a, __float_as_int(y), HI * 0x55, 0xF, 0xA, false));
+}
+
 // the stage values every lane needs: V in all lanes; n, m, h (quad
 // broadcasts) and w (mirror of lane 7) in lane 0
-// (both broadcasts of V run in every lane and a select picks one: a DPP move
-// under a lane-dependent condition would split the wave's exec mask)
+// (V's second move writes the odd banks of four lanes only)
 #define HVC_BCAST8(x)                                            \
     {                                                            \
         const real t_ = oct_mirror(x);                           \
-        const real v_lo_ = quad_bcast<0>(x);                     \
-        const real v_hi_ = quad_bcast<3>(t_);                    \
-        v = q < 4 ? v_lo_ : v_hi_;                               \
+        v = half_bcast<0, 3>(x, t_);                             \
         n1 = quad_bcast<1>(x);                                   \
         m1 = quad_bcast<2>(x);                                   \
         h1 = quad_bcast<3>(x);                                   \
@@ -1264,6 +1269,191 @@ __device__ __forceinline__ void i_dp8_oct(Guard& bad, IState& s, real& xo, real&
     s.V = v; s.n = n1; s.m = m1; s.h = h1; s.w = w1;
     s.Ge = s.Ge * row_e2dt(row);
     s.Gi = s.Gi * row_e5dt(row);
+}
+
+// ---- the octet in the one-thread stepper's arithmetic ----
+// Where a context asks for one thread per neuron but has too few neurons to
+// fill the chip that way, the same numbers come from eight lanes: every
+// product and every fma below is the one the one-thread stepper (i_dp8) is
+// compiled to, so the bits are its bits.
+//
+// The derivative of the lane's own variable but V (i_rates_shared and i_rhs):
+// with E = exp2(fma(v + d, k, k0)) of the lane,
+//   lane 1  an = 0.15 (v + 15) rcp(1 - E)          mirror lane 6: E of bn
+//   lane 2  am = (v + 22) rcp(1 - E e^-0.7)        mirror lane 5: E of bm
+//   lane 3  ah = 0.7 E                             mirror lane 4: rcp(1 + E e^1.1) of bh
+//   lane 7  wInf = rcp(1 + E^4 e^6.8)
+// as one expression r = num (useE ? E : rcp(fma(X, cs, 1))), num =
+// fma(v + d2, c2, c0), X = E or E^4; then k = fma(-s, x, r), s = fma(cm,
+// mirror lane's r, r) or 1 in lane 7.  (Lanes 4-6 carry no variable.)
+struct IOctShared {
+    real d, k, k0, cs, d2, c2, c0, cm, cg, lim;
+    bool useE, pow4;
+    IOctShared() = default;
+    __device__ __forceinline__ explicit IOctShared(int q)
+    {
+        constexpr double L2 = 1.4426950408889634;
+        const bool e10 = q == 1 || q == 2 || q == 4;                     // E = exp(-(v + 15) / 10)
+        d = e10 ? HR(15.0) : HR(0.0);
+        k = e10 ? (real)(-L2 / 10.0)
+                : (q == 5 ? (real)(-L2 / 18.0) : (q == 6 ? (real)(-L2 / 80.0) : (real)(-L2 / 20.0)));
+        k0 = e10 ? HR(0.0)
+                 : (q == 5 ? (real)(-47.0 * L2 / 18.0) : (q == 6 ? (real)(-25.0 * L2 / 80.0) : (real)(-34.0 * L2 / 20.0)));
+        cs = q == 1 ? -HR(1.0) : (q == 2 ? -HR(0.4965853037914095) : (q == 4 ? HR(3.0041660239464334)
+                                                                             : (q == 7 ? HR(897.8472916504176) : HR(0.0))));
+        d2 = q == 1 ? HR(15.0) : HR(22.0);
+        c2 = q == 1 ? HR(0.15) : (q == 2 ? HR(1.0) : HR(0.0));
+        c0 = q == 1 || q == 2 ? HR(0.0) : (q == 3 ? HR(0.7) : HR(1.0));
+        cm = q == 1 ? HR(0.2) : (q == 2 ? HR(40.0) : (q == 3 ? HR(10.0) : HR(0.0)));
+        cg = q == 1 ? HR(1.5) : HR(10.0);                                 // c e of the series (an, am)
+        lim = q == 1 || q == 2 ? HR(0.5) : -HR(1.0);
+        useE = q == 3 || q == 5 || q == 6;
+        pow4 = q == 7;
+    }
+    __device__ __forceinline__ real deriv(int q, real v, real xo) const
+    {
+#pragma clang fp contract(off)
+        const real E = __builtin_amdgcn_exp2f(__builtin_fmaf(v + d, k, k0));
+        const real E2 = E * E;
+        const real X = pow4 ? E2 * E2 : E;
+        const real R = __builtin_amdgcn_rcpf(__builtin_fmaf(X, cs, HR(1.0)));
+        const real vd = v + d2;
+        real r = __builtin_fmaf(vd, c2, c0) * (useE ? E : R);
+        // an, am near their zeros, when a lane of the wave is there
+        const real x = vd * HR(0.1);
+        const bool near = __builtin_fabsf(x) <= lim;
+        if (__any(near)) {
+            asm volatile("");   // (a branch: evaluated always, it lengthens every stage)
+            const real sr = cg * xexpm1_series(x);
+            if (near) r = sr;
+        }
+        const real mr = oct_mirror(r);
+        const real s = q == 7 ? HR(1.0) : __builtin_fmaf(cm, mr, r);
+        return __builtin_fmaf(-s, xo, r);
+    }
+};
+
+// HHI_buffer::DP8_step with eight lanes per neuron in i_dp8's arithmetic; as
+// i_dp8_oct.  A combination of stage derivatives is one chain of fma; where its
+// first two terms have opposite signs, i_dp8 rounds the second term's product
+// for the gates and the first's for V (whose derivative is a negated sum), so
+// V's lane takes the pair exchanged.
+template <class Row>
+__device__ __forceinline__ void i_dp8_shared(IState& s, real& xo, real& xlo, int q, const IOctShared& g, real dt,
+                                             const Row& row)
+{
+#pragma clang fp contract(off)
+    const real x0 = xo;
+    const bool isV = q == 0;
+    real x = xo, v = s.V, n1 = s.n, m1 = s.m, h1 = s.h, w1 = s.w;
+    real e2r[11], e5r[11];
+#pragma unroll
+    for (int k = 0; k < 10; ++k) {
+        e2r[k] = row.e2[kOffDp2 + k];
+        e5r[k] = row.e5[kOffDp2 + k];
+    }
+    e2r[10] = row.e2[kOffDt];
+    e5r[10] = row.e5[kOffDt];
+    auto deriv = [&](real e2, real e5) {
+        const real n2 = n1 * n1;
+        const real gk = __builtin_fmaf(kI_gKdr, n2 * n2, kI_gKHT * w1);
+        real t = __builtin_fmaf(kI_gL, v, -(kI_gL * kI_El));
+        t = __builtin_fmaf((kI_gNa * h1) * (m1 * (m1 * m1)), v - kI_Ena, t);
+        t = __builtin_fmaf(gk, v - kI_Ek, t);
+        t = __builtin_fmaf(s.Ge * e2, v, t);
+        t = __builtin_fmaf(s.Gi * e5, v - kI_Ei, t);
+        const real kg = g.deriv(q, v, x);
+        return isV ? -t : kg;
+    };
+    auto pair = [&](real ca, real ka, real cb, real kb) {   // fma(ka, ca, kb cb), V: fma(kb, cb, ka ca)
+        return __builtin_fmaf(isV ? kb : ka, isV ? cb : ca, (isV ? ka : kb) * (isV ? ca : cb));
+    };
+#define SH_C(n, d) ((real)((double)(n) / (double)(d)))
+#define SH_F(k, c, sum) __builtin_fmaf(k, c, sum)
+    const real k1 = deriv(HR(1.0), HR(1.0));
+    x = __builtin_fmaf(k1, dt * (real)(1.0 / 18), x0);
+    HVC_BCAST8(x)
+    const real k2 = deriv(e2r[0], e5r[0]);
+    x = __builtin_fmaf(SH_F(k2, HR(3.0), k1), dt * (real)(1.0 / 48), x0);
+    HVC_BCAST8(x)
+    const real k3 = deriv(e2r[1], e5r[1]);
+    x = __builtin_fmaf(SH_F(k3, HR(3.0), k1), dt * HR(0.03125), x0);
+    HVC_BCAST8(x)
+    const real k4 = deriv(e2r[2], e5r[2]);
+    x = __builtin_fmaf(SH_F(k4, HR(75.0), pair(HR(20.0), k1, -HR(75.0), k3)), dt * HR(0.015625), x0);
+    HVC_BCAST8(x)
+    const real k5 = deriv(e2r[3], e5r[3]);
+    x = __builtin_fmaf(SH_F(k5, HR(12.0), SH_F(k1, HR(3.0), k4 * HR(15.0))), dt * (real)(1.0 / 80), x0);
+    HVC_BCAST8(x)
+    const real k6 = deriv(e2r[4], e5r[4]);
+    real c = SH_F(k1, SH_C(29443841, 614563906), k4 * SH_C(77736538, 692538347));
+    c = SH_F(k5, -SH_C(28693883, 1125000000), c);
+    c = SH_F(k6, SH_C(23124283, 1800000000), c);
+    x = __builtin_fmaf(c, dt, x0);
+    HVC_BCAST8(x)
+    const real k7 = deriv(e2r[5], e5r[5]);
+    c = SH_F(k1, SH_C(16016141, 946692911), k4 * SH_C(61564180, 158732637));
+    c = SH_F(k5, SH_C(22789713, 633445777), c);
+    c = SH_F(k6, SH_C(545815736, 2771057229), c);
+    c = SH_F(k7, -SH_C(180193667, 1043307555), c);
+    x = __builtin_fmaf(c, dt, x0);
+    HVC_BCAST8(x)
+    const real k8 = deriv(e2r[6], e5r[6]);
+    c = pair(SH_C(39632708, 573591083), k1, -SH_C(433636366, 683701615), k4);
+    c = SH_F(k5, -SH_C(421739975, 2616292301), c);
+    c = SH_F(k6, SH_C(100302831, 723423059), c);
+    c = SH_F(k7, SH_C(790204164, 839813087), c);
+    c = SH_F(k8, SH_C(800635310, 3783071287), c);
+    x = __builtin_fmaf(c, dt, x0);
+    HVC_BCAST8(x)
+    const real k9 = deriv(e2r[7], e5r[7]);
+    c = pair(SH_C(246121993, 1340847787), k1, -SH_C(37695042795, 15268766246), k4);
+    c = SH_F(k5, -SH_C(309121744, 1061227803), c);
+    c = SH_F(k6, -SH_C(12992083, 490766935), c);
+    c = SH_F(k7, SH_C(6005943493, 2108947869), c);
+    c = SH_F(k8, SH_C(393006217, 1396673457), c);
+    c = SH_F(k9, SH_C(123872331, 1001029789), c);
+    x = __builtin_fmaf(c, dt, x0);
+    HVC_BCAST8(x)
+    const real k10 = deriv(e2r[8], e5r[8]);
+    c = pair(SH_C(8478235783, 508512852), k4, SH_C(-1028468189, 846180014), k1);
+    c = SH_F(k5, SH_C(1311729495, 1432422823), c);
+    c = SH_F(k6, -SH_C(10304129995, 1701304382), c);
+    c = SH_F(k7, -SH_C(48777925059, 3047939560), c);
+    c = SH_F(k8, SH_C(15336726248, 1032824649), c);
+    c = SH_F(k9, -SH_C(45442868181, 3398467696), c);
+    c = SH_F(k10, SH_C(3065993473, 597172653), c);
+    x = __builtin_fmaf(c, dt, x0);
+    HVC_BCAST8(x)
+    const real k11 = deriv(e2r[9], e5r[9]);
+    c = pair(SH_C(185892177, 718116043), k1, -SH_C(3185094517, 667107341), k4);
+    c = SH_F(k5, -SH_C(477755414, 1098053517), c);
+    c = SH_F(k6, -SH_C(703635378, 230739211), c);
+    c = SH_F(k7, SH_C(5731566787, 1027545527), c);
+    c = SH_F(k8, SH_C(5232866602, 850066563), c);
+    c = SH_F(k9, -SH_C(4093664535, 808688257), c);
+    c = SH_F(k10, SH_C(3962137247, 1805957418), c);
+    c = SH_F(k11, SH_C(65686358, 487910083), c);
+    x = __builtin_fmaf(c, dt, x0);
+    HVC_BCAST8(x)
+    const real k12 = deriv(e2r[10], e5r[10]);
+    c = pair(SH_C(13451932, 455176623), k1, -SH_C(808719846, 976000145), k6);
+    c = SH_F(k7, SH_C(1757004468, 5645159321), c);
+    c = SH_F(k8, SH_C(656045339, 265891186), c);
+    c = SH_F(k9, -SH_C(3867574721, 1518517206), c);
+    c = SH_F(k10, SH_C(465885868, 322736535), c);
+    c = SH_F(k11, SH_C(53011238, 667516719), c);
+    c = SH_F(k12, SH_C(2, 45), c);
+    const real y = __builtin_fmaf(c, dt, xlo);   // Kahan (HVC_ACC)
+    x = x0 + y;
+    xlo = y - (x - x0);
+    xo = x;
+    HVC_BCAST8(x)
+    s.V = v; s.n = n1; s.m = m1; s.h = h1; s.w = w1;
+    s.Ge = s.Ge * row_e2dt(row);
+    s.Gi = s.Gi * row_e5dt(row);
+#undef SH_C
+#undef SH_F
 }
 #undef HVC_BCAST8
 #endif  // HVC_FP32
