@@ -40,6 +40,28 @@ def test_partly_filled_waves(model, n_ra, n_i):
 
 
 @pytest.mark.parametrize("model", [0, 1])
+@pytest.mark.parametrize("sync_ms", [0.02, 0.35, 0.37, 1.25])
+def test_window_tables(model, sync_ms):
+    """Windows of 1 to 63 steps: the tables that a block of 64 stages with one
+    round of loads (18 steps) and the ones that take more, in FP64 and, against
+    blocks of 256, in FP32."""
+    from unsupervised_growth_amd.engine import Engine
+    from unsupervised_growth_amd.network import random_network
+    net = random_network(20, 12, n_train=4, p_ra2i=0.5, p_i2ra=0.5, seed=5)
+    kw = dict(ra_model=model, ra_poisson=model, sync_ms=sync_ms)
+    _compare(net, 20.0, tuning=dict(integrate_block=64), **kw)
+    states = []
+    for block in (64, 256):
+        with Engine(precision=1, trial_ms=20.0, **kw) as eng:
+            eng.upload(net)
+            eng.set_tuning(integrate_block=block)
+            r = eng.run_trial(mode=0, trial_index=0, first_trial=True, mean_injection_time=5.0, want_state=True)
+            states.append((r.ra_state, r.i_state))
+    for a, b in zip(*states):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("model", [0, 1])
 def test_steps_out_of_the_fast_range(model):
     """Resting potentials far out (gate arguments and voltages beyond the fast
     range, overflowing exponentials) and conductances under which the HVC-I

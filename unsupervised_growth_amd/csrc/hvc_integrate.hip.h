@@ -40,9 +40,9 @@ __device__ __forceinline__ double inbox_sum(const Inbox& ib, int tgt, int n)
 
 // the previous window's sync for one target (NGS:9309-9366): the ordered sum
 // of its inbox, if any, and the inbox emptied
-__device__ __forceinline__ bool inbox_take(const NetDev& nd, const Inbox& ib, int tgt, double& sum)
+// (n: the inbox's count, loaded ahead)
+__device__ __forceinline__ bool inbox_take(const NetDev& nd, const Inbox& ib, int tgt, int n, double& sum)
 {
-    int n = ib.cnt[tgt];
     if (n <= 0) return false;
     if (n > ib.cap) {
         atomicOr(nd.err, (unsigned)kErrInbox);
@@ -164,31 +164,59 @@ struct Win {
     int nsteps;
     __device__ __forceinline__ const WinRow& row(int t) const { return rows[t - t0]; }
     __device__ __forceinline__ double clk(int t) const { return clock[t - t0 + 1]; }
-    // copy the tables into LDS (every thread of the block, after it has issued
-    // its state loads, so their latencies overlap)
-    __device__ __forceinline__ void stage(const NetDev& nd) const
+    // Copy the tables into LDS, by every thread of the block.  load() issues
+    // kStagePieces reads of 16 bytes a thread (all of an 18-step window's rows
+    // in blocks of 64) and store() writes them, so that the tables arrive
+    // together with the neuron's state, which the caller loads before, in one
+    // memory latency (the L2s are cold after a kernel boundary); the loop of
+    // 8-byte copies waited six times.  From a wave's start to its first step,
+    // with the neuron's loads ahead of the tables' and kernarg_touch, FP64
+    // HVC-I octets: 9 900 -> 2 550 cycles, 2.8 us of a 47 us window.
+    typedef double Piece __attribute__((ext_vector_type(2)));
+    static constexpr int kRowPieces = (int)(sizeof(DecayRow) / sizeof(Piece));
+    struct Tables {
+        Piece v[kStagePieces];
+        double c;
+    };
+    __device__ __forceinline__ const Piece* pieces(const NetDev& nd) const
     {
-        const DecayRow* grow = (const DecayRow*)nd.decay + t0;
-        WinRow* rl = (WinRow*)lds;
+        return (const Piece*)((const DecayRow*)nd.decay + t0);
+    }
+    __device__ __forceinline__ Tables load(const NetDev& nd) const
+    {
+        Tables t;
+        const int last = nsteps * kRowPieces - 1;
+#pragma unroll
+        for (int u = 0; u < kStagePieces; ++u) t.v[u] = pieces(nd)[min((int)(threadIdx.x + u * blockDim.x), last)];
+        t.c = nd.clock[t0 - 1 + min((int)threadIdx.x, nsteps)];
+        return t;
+    }
+    __device__ __forceinline__ void put(int p, Piece v) const
+    {
 #ifdef HVC_FP32
-        for (int k = threadIdx.x; k < nsteps * kNumOffsets; k += blockDim.x) {
-            const int r = k / kNumOffsets, o = k - r * kNumOffsets;
-            rl[r].e5[o] = (float)grow[r].e5[o];
-            rl[r].e2[o] = (float)grow[r].e2[o];
-            if (o == kOffDt) {
-                rl[r].e5dt = grow[r].e5[o];
-                rl[r].e2dt = grow[r].e2[o];
-            }
-        }
+        const int r = p / kRowPieces, o = p - r * kRowPieces;
+        WinRow* row = (WinRow*)lds + r;
+        ((float2*)row)[o] = make_float2((float)v.x, (float)v.y);   // e5, then e2
+        if (o == 0) row->e5dt = v.x;
+        if (o == kRowPieces / 2) row->e2dt = v.x;
 #else
-        constexpr int kRowWords = (int)(sizeof(DecayRow) / sizeof(double));
-        for (int k = threadIdx.x; k < nsteps * kRowWords; k += blockDim.x) lds[k] = ((const double*)grow)[k];
+        ((Piece*)lds)[p] = v;
 #endif
-        double* wc = (double*)(rl + nsteps);
-        for (int k = threadIdx.x; k <= nsteps; k += blockDim.x) wc[k] = nd.clock[t0 - 1 + k];
+    }
+    __device__ __forceinline__ void store(const NetDev& nd, const Tables& t) const
+    {
+        const int n = nsteps * kRowPieces;
+        double* wc = (double*)((WinRow*)lds + nsteps);
+#pragma unroll
+        for (int u = 0; u < kStagePieces; ++u) put(min((int)(threadIdx.x + u * blockDim.x), n - 1), t.v[u]);
+        wc[min((int)threadIdx.x, nsteps)] = t.c;
+        for (int p = threadIdx.x + kStagePieces * blockDim.x; p < n; p += blockDim.x) put(p, pieces(nd)[p]);
+        for (int k = threadIdx.x + blockDim.x; k <= nsteps; k += blockDim.x) wc[k] = nd.clock[t0 - 1 + k];
         __syncthreads();
     }
+    __device__ __forceinline__ void stage(const NetDev& nd) const { store(nd, load(nd)); }
 };
+static_assert(kOffDt == 0 && kNumOffsets % 2 == 0, "put() finds the whole-step factors at the start of each half row");
 
 // The neuron's next two noise events of the chunk (lists are generated by
 // k_noise_events).  take() applies every event of step t, in list order; the
@@ -302,13 +330,13 @@ struct RAPosts {
     double last;      // the latest one's time (count > 0)
 };
 // post events detected in the previous window become visible now (NGS:9385-9386);
-// lead: the lane that keeps neuron ii's events
+// lead: the lane that keeps neuron ii's events; count, pend: the neuron's
+// post_cnt and post_pend, loaded ahead
 __device__ __forceinline__ RAPosts ra_posts_begin(const NetDev& nd, const Win& win, int growth, int ii, int t0,
-                                                  bool lead)
+                                                  bool lead, int count, int pend)
 {
-    RAPosts p{growth, nd.post_cnt[ii], 0.0};
+    RAPosts p{growth, count, 0.0};
     if (growth && lead) {
-        int pend = nd.post_pend[ii];
         if (pend > 0) {
             double cs = win.clk(t0 - 1);
             for (int q = 0; q < pend; ++q) {
@@ -394,32 +422,37 @@ __device__ void integrate_ra(const NetDev& nd, const Win& win, int slot, int t0,
     HVC_LOAD(s, Vs, nd.ra[0][ii]) HVC_LOAD(s, Vd, nd.ra[1][ii]) HVC_LOAD(s, n, nd.ra[2][ii])
     HVC_LOAD(s, l, nd.ra[3][ii]) HVC_LOAD(s, h, nd.ra[4][ii]) HVC_LOAD(s, r, nd.ra[5][ii])
     HVC_LOAD(s, c, nd.ra[6][ii]) HVC_LOAD(s, Ca, nd.ra[7][ii])
-    win.stage(nd);
-    // the previous window's sync: raiseI (Gi_d += G), raiseExcWeight (Ge_d += w / Ad)
     double ge_d = nd.ra[10][ii], gi_d = nd.ra[11][ii];
+    s.Ge_s = nd.ra[8][ii]; s.Gi_s = nd.ra[9][ii];
+    const int flags = nd.ra_flags[ii];
+    const real el = (real)nd.EL[ii], gca = (real)nd.GCa[ii];
+    const int kick = nd.kick_step[ii];
+    const int n_gi = nd.in_gi_ra.cnt[ii], n_ge = nd.in_ge_ra.cnt[ii];
+    const int post_cnt = nd.post_cnt[ii], post_pend = nd.post_pend[ii];
+    const bool poisson = MODEL == 1 && nd.ra_poisson;
+    const int ev_pos = poisson ? nd.ra_ev_pos[ii] : 0;
+    const Win::Tables tab = win.load(nd);
+    const NoiseId sid = ra_noise_id(nd, ii);
+    NoiseCursor nc;
+    if (poisson)
+        nc.open(nd.ra_ev + (size_t)ii * nd.ev_cap, ev_pos);
+    else
+        nc.none();
+    win.store(nd, tab);
+    // the previous window's sync: raiseI (Gi_d += G), raiseExcWeight (Ge_d += w / Ad)
     if (live && leader) {
         double sum;
-        if (inbox_take(nd, nd.in_gi_ra, i, sum)) gi_d += sum;
-        if (inbox_take(nd, nd.in_ge_ra, i, sum)) ge_d += HVC_CDIV(sum, 10000);
+        if (inbox_take(nd, nd.in_gi_ra, i, n_gi, sum)) gi_d += sum;
+        if (inbox_take(nd, nd.in_ge_ra, i, n_ge, sum)) ge_d += HVC_CDIV(sum, 10000);
     }
     if constexpr (LANES) {
         ge_d = quad_bcast<0>(ge_d);
         gi_d = quad_bcast<0>(gi_d);
     }
-    s.Ge_s = nd.ra[8][ii]; s.Gi_s = nd.ra[9][ii]; s.Ge_d = ge_d; s.Gi_d = gi_d;
-    int flags = nd.ra_flags[ii];
+    s.Ge_d = ge_d; s.Gi_d = gi_d;
     int fs = flags & 1, fd = (flags >> 1) & 1;
-    const real el = (real)nd.EL[ii], gca = (real)nd.GCa[ii];
-    const int kick = nd.kick_step[ii];
 
-    const RAPosts posts = ra_posts_begin(nd, win, growth, ii, t0, live && leader);
-
-    const NoiseId sid = ra_noise_id(nd, ii);
-    NoiseCursor nc;
-    if (MODEL == 1 && nd.ra_poisson)
-        nc.open(nd.ra_ev + (size_t)ii * nd.ev_cap, nd.ra_ev_pos[ii]);
-    else
-        nc.none();
+    const RAPosts posts = ra_posts_begin(nd, win, growth, ii, t0, live && leader, post_cnt, post_pend);
 
     uint64_t smask = 0, dmask = 0;
     for (int t = t0; t <= t1; ++t) {
@@ -471,20 +504,23 @@ __device__ void integrate_i_thread(const NetDev& nd, const Win& win, int i, int 
     HVC_LOAD(s, V, nd.in[0][ii]) HVC_LOAD(s, n, nd.in[1][ii]) HVC_LOAD(s, m, nd.in[2][ii])
     HVC_LOAD(s, h, nd.in[3][ii]) HVC_LOAD(s, w, nd.in[4][ii])
     const int listed = nd.wl_on ? nd.wl_mark[2][ii] : 0;
-    win.stage(nd);
-    // the previous window's sync: HHI raiseE (Ge += G)
     double ge = nd.in[5][ii];
-    if (live) {
-        double sum;
-        if (inbox_take(nd, nd.in_ge_i, i, sum)) ge += sum;
-    }
-    s.Ge = ge; s.Gi = nd.in[6][ii];
+    s.Gi = nd.in[6][ii];
     int flag = nd.i_flag[ii];
+    const int n_in = nd.in_ge_i.cnt[ii], ev_pos = nd.i_poisson ? nd.i_ev_pos[ii] : 0;
+    const Win::Tables tab = win.load(nd);
     NoiseCursor nc;
     if (nd.i_poisson)
-        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, nd.i_ev_pos[ii]);
+        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, ev_pos);
     else
         nc.none();
+    win.store(nd, tab);
+    // the previous window's sync: HHI raiseE (Ge += G)
+    if (live) {
+        double sum;
+        if (inbox_take(nd, nd.in_ge_i, i, n_in, sum)) ge += sum;
+    }
+    s.Ge = ge;
     uint64_t mask = 0;
     for (int t = t0; t <= t1; ++t) {
         int f = i_state_check(s.V, flag);
@@ -531,21 +567,24 @@ __device__ void integrate_i_lanes(const NetDev& nd, const Win& win, int wave, in
     HVC_LOAD(s, V, nd.in[0][ii]) HVC_LOAD(s, n, nd.in[1][ii]) HVC_LOAD(s, m, nd.in[2][ii])
     HVC_LOAD(s, h, nd.in[3][ii]) HVC_LOAD(s, w, nd.in[4][ii])
     const int listed = nd.wl_on ? nd.wl_mark[2][ii] : 0;
-    win.stage(nd);
-    // the previous window's sync: HHI raiseE (Ge += G), by the group's first lane
     double ge = nd.in[5][ii];
-    if (live && role == 0) {
-        double sum;
-        if (inbox_take(nd, nd.in_ge_i, i, sum)) ge += sum;
-    }
-    ge = __shfl(ge, base);
-    s.Ge = ge; s.Gi = nd.in[6][ii];
+    s.Gi = nd.in[6][ii];
     int flag = nd.i_flag[ii];
+    const int n_in = nd.in_ge_i.cnt[ii], ev_pos = nd.i_poisson ? nd.i_ev_pos[ii] : 0;
+    const Win::Tables tab = win.load(nd);
     NoiseCursor nc;
     if (nd.i_poisson)
-        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, nd.i_ev_pos[ii]);
+        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, ev_pos);
     else
         nc.none();
+    win.store(nd, tab);
+    // the previous window's sync: HHI raiseE (Ge += G), by the group's first lane
+    if (live && role == 0) {
+        double sum;
+        if (inbox_take(nd, nd.in_ge_i, i, n_in, sum)) ge += sum;
+    }
+    ge = __shfl(ge, base);
+    s.Ge = ge;
     // low part of this lane's own variable (FP32 form; zero in FP64)
     real xlo = 0;
 #ifdef HVC_FP32
@@ -597,21 +636,24 @@ __device__ void integrate_i_quad(const NetDev& nd, const Win& win, int wave, int
     HVC_LOAD(s, V, nd.in[0][ii]) HVC_LOAD(s, n, nd.in[1][ii]) HVC_LOAD(s, m, nd.in[2][ii])
     HVC_LOAD(s, h, nd.in[3][ii]) HVC_LOAD(s, w, nd.in[4][ii])
     const int listed = nd.wl_on ? nd.wl_mark[2][ii] : 0;
-    win.stage(nd);
-    // the previous window's sync: HHI raiseE (Ge += G), by the quad's first lane
     double ge = nd.in[5][ii];
-    if (live && role == 0) {
-        double sum;
-        if (inbox_take(nd, nd.in_ge_i, i, sum)) ge += sum;
-    }
-    ge = quad_bcast<0>(ge);
-    s.Ge = ge; s.Gi = nd.in[6][ii];
+    s.Gi = nd.in[6][ii];
     int flag = nd.i_flag[ii];
+    const int n_in = nd.in_ge_i.cnt[ii], ev_pos = nd.i_poisson ? nd.i_ev_pos[ii] : 0;
+    const Win::Tables tab = win.load(nd);
     NoiseCursor nc;
     if (nd.i_poisson)
-        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, nd.i_ev_pos[ii]);
+        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, ev_pos);
     else
         nc.none();
+    win.store(nd, tab);
+    // the previous window's sync: HHI raiseE (Ge += G), by the quad's first lane
+    if (live && role == 0) {
+        double sum;
+        if (inbox_take(nd, nd.in_ge_i, i, n_in, sum)) ge += sum;
+    }
+    ge = quad_bcast<0>(ge);
+    s.Ge = ge;
     // low parts of this lane's variable and of w (FP32 form; zero in FP64)
     real xlo = 0, wlo = 0;
 #ifdef HVC_FP32
@@ -666,30 +708,33 @@ __device__ void integrate_i_oct(const NetDev& nd, const Win& win, int wave, int 
     const int i = wave * kINeuronsPerOctWave + (lane >> 3);
     const bool live = i < nd.n_i && (!nd.net_live || nd.net_live[nd.i_net[i]]);
     const int ii = live ? i : 0;
-    Gate g;
-    i_oct_gate(g, q);
     // the lane's own variable: V (lane 0), n (1, 6), m (2, 5), h (3, 4), w (7)
     const int var = q == 0 ? 0 : (q == 1 || q == 6 ? 1 : (q == 2 || q == 5 ? 2 : (q == 7 ? 4 : 3)));
     IState s;
     HVC_LOAD(s, V, nd.in[0][ii]) HVC_LOAD(s, n, nd.in[1][ii]) HVC_LOAD(s, m, nd.in[2][ii])
     HVC_LOAD(s, h, nd.in[3][ii]) HVC_LOAD(s, w, nd.in[4][ii])
     const int listed = nd.wl_on ? nd.wl_mark[2][ii] : 0;
-    win.stage(nd);
-    // the previous window's sync: HHI raiseE (Ge += G), by the octet's first lane
     double ge = nd.in[5][ii];
+    s.Gi = nd.in[6][ii];
+    int flag = nd.i_flag[ii];
+    const int n_in = nd.in_ge_i.cnt[ii], ev_pos = nd.i_poisson ? nd.i_ev_pos[ii] : 0;
+    const Win::Tables tab = win.load(nd);
+    Gate g;
+    i_oct_gate(g, q);
+    NoiseCursor nc;
+    if (nd.i_poisson)
+        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, ev_pos);
+    else
+        nc.none();
+    win.store(nd, tab);
+    // the previous window's sync: HHI raiseE (Ge += G), by the octet's first lane
     if (live && q == 0) {
         double sum;
-        if (inbox_take(nd, nd.in_ge_i, i, sum)) ge += sum;
+        if (inbox_take(nd, nd.in_ge_i, i, n_in, sum)) ge += sum;
     }
     const double ge_lo = quad_bcast<0>(ge), ge_hi = quad_bcast<3>(oct_mirror(ge));
     ge = q < 4 ? ge_lo : ge_hi;
-    s.Ge = ge; s.Gi = nd.in[6][ii];
-    int flag = nd.i_flag[ii];
-    NoiseCursor nc;
-    if (nd.i_poisson)
-        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, nd.i_ev_pos[ii]);
-    else
-        nc.none();
+    s.Ge = ge;
     real xo = var == 0 ? s.V : (var == 1 ? s.n : (var == 2 ? s.m : (var == 3 ? s.h : s.w)));
     real xlo = 0;
     xlo = var == 0 ? s.V_lo : (var == 1 ? s.n_lo : (var == 2 ? s.m_lo : (var == 3 ? s.h_lo : s.w_lo)));
@@ -748,29 +793,34 @@ __device__ void integrate_i_oct(const NetDev& nd, const Win& win, const OctLds& 
     const int i = wave * kINeuronsPerOctWave + (lane >> 3);
     const bool live = i < nd.n_i && (!nd.net_live || nd.net_live[nd.i_net[i]]);
     const int ii = live ? i : 0;
+    // everything the window reads of the neuron and its tables, issued together;
+    // the lane's constants are made while it is on its way
     double* xp = state_array<7>(nd.in, i_oct_var(q));
     double x = xp[ii];
-    if (q > 3 && q < 7) x = 1 - x;
     const int listed = nd.wl_on ? nd.wl_mark[2][ii] : 0;
     double Ge = nd.in[5][ii], Gi = nd.in[6][ii];
     int flag = nd.i_flag[ii];
+    const int n_in = nd.in_ge_i.cnt[ii], ev_pos = nd.i_poisson ? nd.i_ev_pos[ii] : 0;
+    const Win::Tables tab = win.load(nd);
+    const ExpPair ex = exp_table_load();
     const IOctLane L = i_oct_lane(q, lds.exp);
-    stage_exp_table(lds.exp);
-    win.stage(nd);
+    Dp8Consts C;
+    dp8_pin(C);
+    NoiseCursor nc;
+    if (nd.i_poisson)
+        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, ev_pos);
+    else
+        nc.none();
+    exp_table_store(lds.exp, ex);
+    win.store(nd, tab);
+    if (q > 3 && q < 7) x = 1 - x;
     // the previous window's sync: HHI raiseE (Ge += G); only the octet's first
     // lane uses the conductances
     if (live && q == 0) {
         double sum;
-        if (inbox_take(nd, nd.in_ge_i, i, sum)) Ge += sum;
+        if (inbox_take(nd, nd.in_ge_i, i, n_in, sum)) Ge += sum;
     }
-    NoiseCursor nc;
-    if (nd.i_poisson)
-        nc.open(nd.i_ev + (size_t)ii * nd.ev_cap, nd.i_ev_pos[ii]);
-    else
-        nc.none();
     const double dt = nd.dt;
-    Dp8Consts C;
-    dp8_pin(C);
     uint64_t mask = 0;
     for (int t = t0; t <= t1; ++t) {
         const int f = i_state_check(x, flag);   // of V in lane 0
@@ -838,27 +888,34 @@ __device__ void integrate_ra_oct(const NetDev& nd, const Win& win, const OctLds&
     const int flags = nd.ra_flags[ii];
     int flag = q == 0 ? flags & 1 : (flags >> 1) & 1;
     const int kick = nd.kick_step[ii];
+    const int n_gi = nd.in_gi_ra.cnt[ii], n_ge = nd.in_ge_ra.cnt[ii];
+    const int post_cnt = nd.post_cnt[ii], post_pend = nd.post_pend[ii];
+    const bool poisson = MODEL == 1 && nd.ra_poisson;
+    const int ev_pos = poisson ? nd.ra_ev_pos[ii] : 0;
+    const double EL = nd.EL[ii], GCa = nd.GCa[ii];
+    const Win::Tables tab = win.load(nd);
+    const ExpPair ex = exp_table_load();
     const NoiseId sid = ra_noise_id(nd, ii);
-    const RAOctLane L = ra_oct_lane<MODEL>(q, nd.EL[ii], nd.GCa[ii], nd.mu_term_s, nd.mu_term_d, lds.exp);
+    const RAOctLane L = ra_oct_lane<MODEL>(q, EL, GCa, nd.mu_term_s, nd.mu_term_d, lds.exp);
     uint8_t* at = lds.at + (threadIdx.x >> 3) * (2 * kMaxWindowSteps);
-    stage_exp_table(lds.exp);
+    exp_table_store(lds.exp, ex);
+    NoiseCursor nc;
     if constexpr (MODEL == 0) {
         stage_noise_rows(lds.noise, nd.sq_sig_s, nd.sq_sig_d);
         noise_window(at, q, sid, t0, t1 - t0 + 1);
     }
-    win.stage(nd);
+    if (poisson)
+        nc.open(nd.ra_ev + (size_t)ii * nd.ev_cap, ev_pos);
+    else
+        nc.none();
+    win.store(nd, tab);
     // the previous window's sync: raiseExcWeight (Ge_d += w / Ad), raiseI (Gi_d += G)
     if (dend) {
         double sum;
-        if (inbox_take(nd, nd.in_gi_ra, i, sum)) GB += sum;
-        if (inbox_take(nd, nd.in_ge_ra, i, sum)) GA += HVC_CDIV(sum, 10000);
+        if (inbox_take(nd, nd.in_gi_ra, i, n_gi, sum)) GB += sum;
+        if (inbox_take(nd, nd.in_ge_ra, i, n_ge, sum)) GA += HVC_CDIV(sum, 10000);
     }
-    const RAPosts posts = ra_posts_begin(nd, win, growth, ii, t0, soma);
-    NoiseCursor nc;
-    if (MODEL == 1 && nd.ra_poisson)
-        nc.open(nd.ra_ev + (size_t)ii * nd.ev_cap, nd.ra_ev_pos[ii]);
-    else
-        nc.none();
+    const RAPosts posts = ra_posts_begin(nd, win, growth, ii, t0, soma, post_cnt, post_pend);
     const double dt = nd.dt;
     uint64_t mask = 0;   // somatic spikes in lane 0, dendritic ones in lane 5
     for (int t = t0; t <= t1; ++t) {
@@ -894,6 +951,20 @@ __device__ void integrate_ra_oct(const NetDev& nd, const Win& win, const OctLds&
 }
 #endif
 
+// Reads one word of every 64-byte line of the launch arguments, all at once:
+// the neuron functions read them in several rounds, and the first wave of a
+// compute unit would wait for a line of them in each.
+__device__ __forceinline__ void kernarg_touch(const NetDev& nd)
+{
+    constexpr int kLines = (int)(sizeof(NetDev) / 64);
+    const int* w = (const int*)&nd;
+    int x[kLines];
+#pragma unroll
+    for (int k = 0; k < kLines; ++k) x[k] = w[16 * k];
+#pragma unroll
+    for (int k = 0; k < kLines; ++k) asm volatile("" ::"s"(x[k]));
+}
+
 // blocks [0, iblocks) integrate HVC-I, the next rblocks HVC-RA, in the layout
 // of LANES; any blocks after them run the previous window's sync-point STDP
 // (one row per thread, sa).
@@ -912,9 +983,10 @@ __global__ __launch_bounds__(256) void k_integrate(NetDev nd, int t0, int t1, in
         stdp_block(nd, sa, ((int)blockIdx.x - iblocks - rblocks) * blockDim.x, stdp_slice, &stdp_count);
         return;
     }
+    kernarg_touch(nd);
     // the window's decay rows and clock, staged in LDS (dynamic shared memory of
     // win_bytes(t1 - t0 + 1) bytes) by Win::stage in the neuron functions
-    extern __shared__ double win_lds[];
+    extern __shared__ __attribute__((aligned(16))) double win_lds[];
     const int nsteps = t1 - t0 + 1;
     const Win win{(const WinRow*)win_lds, (const double*)((const WinRow*)win_lds + nsteps), t0, win_lds, nsteps};
     const int iwave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -1006,7 +1078,7 @@ __global__ __launch_bounds__(64) void k_trace_ra(NetDev nd, int n, int n_steps, 
                                                  const double* GCa, const double* kick, const double* exc_w,
                                                  const double* inh_g, double* out, uint8_t* fired_out)
 {
-    extern __shared__ double trace_lds[];
+    extern __shared__ __attribute__((aligned(16))) double trace_lds[];
     const int k0 = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = k0 < n;
     const int k = live ? k0 : n - 1;
@@ -1062,7 +1134,7 @@ __global__ __launch_bounds__(64) void k_trace_i(NetDev nd, int n, int n_steps, i
                                                 const double* exc_g, const double* inh_g, double* out,
                                                 uint8_t* fired_out)
 {
-    extern __shared__ double trace_lds[];
+    extern __shared__ __attribute__((aligned(16))) double trace_lds[];
     const int k0 = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = k0 < n;
     const int k = live ? k0 : n - 1;
@@ -1126,7 +1198,7 @@ __global__ __launch_bounds__(64) void k_trace_ra_oct(NetDev nd, int n, int n_ste
                                                      const double* GCa, const double* kick, const double* exc_w,
                                                      const double* inh_g, double* out, uint8_t* fired_out)
 {
-    extern __shared__ double trace_lds[];
+    extern __shared__ __attribute__((aligned(16))) double trace_lds[];
     __shared__ ExpPair exp_tab[64];
     __shared__ RANoise noise_rows[MODEL == 0 ? kNoiseRows : 1];
     __shared__ uint8_t noise_at[8 * 2 * kTraceChunk];
@@ -1134,7 +1206,7 @@ __global__ __launch_bounds__(64) void k_trace_ra_oct(NetDev nd, int n, int n_ste
     const int lane = threadIdx.x, q = lane & 7, g = lane >> 3;
     const bool live = (int)blockIdx.x * 8 + g < n;
     const int k = live ? blockIdx.x * 8 + g : n - 1;
-    stage_exp_table(exp_tab);
+    exp_table_store(exp_tab, exp_table_load());
     if constexpr (MODEL == 0) stage_noise_rows(noise_rows, nd.sq_sig_s, nd.sq_sig_d);
     const RAOctLane L = ra_oct_lane<MODEL>(q, EL[k], GCa[k], nd.mu_term_s, nd.mu_term_d, exp_tab);
     // HH2_test::set_to_rest (HH2_test.cpp:196-205), by state variable
@@ -1196,13 +1268,13 @@ __global__ __launch_bounds__(64) void k_trace_i_oct(NetDev nd, int n, int n_step
                                                     const double* exc_g, const double* inh_g, double* out,
                                                     uint8_t* fired_out)
 {
-    extern __shared__ double trace_lds[];
+    extern __shared__ __attribute__((aligned(16))) double trace_lds[];
     __shared__ ExpPair exp_tab[64];
     __shared__ double in_exc[8 * kTraceChunk], in_inh[8 * kTraceChunk];
     const int lane = threadIdx.x, q = lane & 7, g = lane >> 3;
     const bool live = (int)blockIdx.x * 8 + g < n;
     const int k = live ? blockIdx.x * 8 + g : n - 1;
-    stage_exp_table(exp_tab);
+    exp_table_store(exp_tab, exp_table_load());
     const IOctLane L = i_oct_lane(q, exp_tab);
     // HHI_buffer::set_to_rest (HHI_buffer.cpp:181-185), by state variable; the
     // mirror lanes 4-6 carry 1 - x

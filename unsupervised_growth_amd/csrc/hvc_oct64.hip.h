@@ -18,8 +18,8 @@
 //
 // Instructions per step and wave: HVC-I 1 350 (2 400 before, in 96 pieces
 // between lane-dependent branches), HVC-RA Debraband 640 (one thread per
-// neuron 5 600).  k_integrate per window, before and now: Debraband 100 -> 44
-// us at 300 + 30 neurons and 99 -> 45 us at 5 003 + 1 377, RK4 67 -> 45 us at
+// neuron 5 600).  k_integrate per window, before and now: Debraband 100 -> 41
+// us at 300 + 30 neurons and 99 -> 42 us at 5 003 + 1 377, RK4 67 -> 42 us at
 // 2 000 + 550.  Now the HVC-I wave sets the window; its instructions take 5.2
 // cycles each on average.
 //
@@ -56,10 +56,13 @@ __device__ __forceinline__ void every_lane(double& x) { asm volatile("" : "+v"(x
 typedef double ExpPair __attribute__((ext_vector_type(2)));
 constexpr int kExpTabBytes = 64 * (int)sizeof(ExpPair);
 
-__device__ __forceinline__ void stage_exp_table(ExpPair* tab)
+// one entry per thread (blocks of 64 threads or more)
+__device__ __forceinline__ ExpPair exp_table_load()
 {
-    for (int j = threadIdx.x; j < 64; j += blockDim.x) tab[j] = ExpPair{kExp2Table[2 * j], kExp2Table[2 * j + 1]};
+    const double* e = kExp2Table + 2 * (threadIdx.x & 63);
+    return ExpPair{e[0], e[1]};
 }
+__device__ __forceinline__ void exp_table_store(ExpPair* tab, ExpPair v) { tab[threadIdx.x & 63] = v; }
 
 // dexp for |x| <= 700 (no clamp needed, results normal): the same operations
 __device__ __forceinline__ double exp_inrange(double x, const ExpPair* tab)
@@ -128,10 +131,13 @@ __device__ __forceinline__ double qconst(double a, double B)
 struct LaneDiv {
     double B, hi, lo;
 };
-__device__ __forceinline__ LaneDiv lane_div(double B)
+constexpr double upper_half(double x) { return 134217729.0 * x - (134217729.0 * x - x); }
+constexpr LaneDiv lane_div(double B)
 {
-    const double hi = 1.0 / B;
-    return LaneDiv{B, hi, __builtin_fma(-B, hi, 1.0) / B};
+    // 1 - B hi exactly, the product as p + e (Dekker 1971, Numer. Math. 18)
+    const double hi = 1.0 / B, Bh = upper_half(B), Bl = B - Bh, hh = upper_half(hi), hl = hi - hh;
+    const double p = B * hi, e = ((Bh * hh - p) + Bh * hl + Bl * hh) + Bl * hl;
+    return LaneDiv{B, hi, ((1.0 - p) - e) / B};
 }
 template <bool EXACT>
 __device__ __forceinline__ double qlane(double a, const LaneDiv& d)
@@ -148,23 +154,37 @@ __device__ __forceinline__ double qlane(double a, const LaneDiv& d)
 // r (1 + cx x) - b x with the mirror lane's rate b: cx = -1 for the gates; for
 // w, cx = 0 and b = 1 (lane 0's rate), which is wInf - w exactly.
 // ---------------------------------------------------------------------------
-struct IOctLane {
-    int q;
-    GateSlot g;             // the gate as the EXACT step evaluates it
+struct IOctConst {
     double d;               // rate = fma(cA, v + d, cC) / fma(sg, E, 1) * fma(cB, E, sB),
     LaneDiv e;              // E = exp((v + d) / e), e negative
     double cA, cC, sg, cB, sB;
     double cx;
+};
+// the gates of kIOctGates: type 0 (A), 1 (B) or 2 (C), c, d, e
+constexpr IOctConst i_oct_const(int type, double c, double d, double e, double cx = -1.0)
+{
+    return IOctConst{d, lane_div(-e), type == 0 ? c : 0.0, type == 0 ? 0.0 : (type == 2 ? c : 1.0),
+                     type == 0 ? -1.0 : (type == 1 ? 0.0 : 1.0), type == 1 ? c : 0.0, type == 1 ? 0.0 : 1.0, cx};
+}
+static __constant__ IOctConst kIOctConsts[8] = {
+    IOctConst{0.0, lane_div(-10.0), 0.0, 1.0, 0.0, 0.0, 1.0, -1.0},   // V: rate 1
+    i_oct_const(0, 0.15, 15.0, 10.0), i_oct_const(0, 1.0, 22.0, 10.0), i_oct_const(1, 0.7, 34.0, 20.0),
+    i_oct_const(2, 10.0, 4.0, 10.0), i_oct_const(1, 40.0, 47.0, 18.0), i_oct_const(1, 0.2, 25.0, 80.0),
+    i_oct_const(2, 1.0, 0.0, 5.0, 0.0)};
+struct IOctLane : IOctConst {
+    int q;
     const ExpPair* tab;
 };
 
+// (a lane's constants come from memory with its state: as selects among
+// literals they became a tree of branches)
 __device__ __forceinline__ IOctLane i_oct_lane(int q, const ExpPair* tab)
 {
-    const GateSlot g = kIOctGates[q];
-    const bool A = g.type == 0, B = g.type == 1, C = g.type == 2;
-    const bool rate1 = q == 0;   // lane 0: rate 1
-    return IOctLane{q, g, g.d, lane_div(-g.e), A ? g.c : 0.0, A ? 0.0 : (C ? g.c : 1.0), A ? -1.0 : (B ? 0.0 : 1.0),
-                    B && !rate1 ? g.c : 0.0, B && !rate1 ? 0.0 : 1.0, q == 7 ? 0.0 : -1.0, tab};
+    IOctLane L;
+    (IOctConst&)L = kIOctConsts[q];
+    L.q = q;
+    L.tab = tab;
+    return L;
 }
 
 template <bool EXACT>
@@ -172,10 +192,11 @@ __device__ __forceinline__ double i_oct_rate(const IOctLane& L, double v)
 {
     const double vd = v + L.d;
     if constexpr (EXACT) {
-        const double E = dexp(-vd / L.g.e);
-        const double num = L.g.type == 0 ? L.g.c * vd : L.g.c;
-        const double den = L.g.type == 0 ? 1 - E : 1 + E;
-        return L.g.type == 1 ? L.g.c * E : num / den;
+        const GateSlot& g = kIOctGates[L.q];
+        const double E = dexp(-vd / g.e);
+        const double num = g.type == 0 ? g.c * vd : g.c;
+        const double den = g.type == 0 ? 1 - E : 1 + E;
+        return g.type == 1 ? g.c * E : num / den;
     } else {
         const double E = exp_inrange(qlane<false>(vd, L.e), L.tab);
         const double q = div_inrange(__builtin_fma(L.cA, vd, L.cC), __builtin_fma(L.sg, E, 1.0));
@@ -239,7 +260,7 @@ constexpr double kDp8D[kDp8Terms] = {
 // the compiler would otherwise build from two scalar moves each at every use
 // (227 of a step's 1 490 instructions), the first kDp8Pinned terms keep in
 // vector registers (the count that leaves two waves to a SIMD).
-constexpr int kDp8Pinned = 22;
+constexpr int kDp8Pinned = 21;
 struct Dp8Consts {
     double n[kDp8Pinned], hi[kDp8Pinned], lo[kDp8Pinned];
 };
@@ -393,29 +414,36 @@ struct RAOctLane {
     const ExpPair* tab;
 };
 
+struct RAOctConst {
+    double d;
+    LaneDiv e;
+    double g0, c, den;       // den: the Debraband model's (the RK4 model's c has 10)
+    LaneDiv R;
+};
+static __constant__ RAOctConst kRAOctConsts[8] = {
+    {30.0, lane_div(-9.5), 0.0, 1.0, 1.0, lane_div(275000.0)},     // mInf
+    {35.0, lane_div(-10.0), 0.0, 1.0, 1.0, lane_div(275000.0)},    // nInf
+    {45.0, lane_div(7.0), 0.0, 1.0, 1.0, lane_div(275000.0)},      // hInf
+    {40.0, lane_div(-5.0), 0.0, 1.0, 10.0, lane_div(275000.0)},    // lInf
+    {5.0, lane_div(-10.0), 0.0, 1.0, 1.0, lane_div(550000.0)},     // rInf
+    {40.5, lane_div(6.0), 0.1, 0.75, 1.0, lane_div(550000.0)},     // tauH
+    {27.0, lane_div(15.0), 0.1, 0.5, 1.0, lane_div(550000.0)},     // tauN
+    {-10.0, lane_div(-7.0), 0.0, 1.0, 15.0, lane_div(550000.0)}};  // cInf
+
 template <int MODEL>
 __device__ __forceinline__ RAOctLane ra_oct_lane(int q, double EL, double GCa, double mu_s, double mu_d,
                                                  const ExpPair* tab)
 {
-    //                      mInf   nInf   hInf  lInf   rInf   tauH  tauN  cInf
-    constexpr double d[8] = {30.0, 35.0, 45.0, 40.0, 5.0, 40.5, 27.0, -10.0};
-    constexpr double e[8] = {-9.5, -10.0, 7.0, -5.0, -10.0, 6.0, 15.0, -7.0};
-    constexpr double den[8] = {1.0, 1.0, 1.0, 10.0, 1.0, 1.0, 1.0, MODEL == 0 ? 15.0 : 10.0};
-    auto pick = [&](const double (&t)[8]) {
-        double x = t[0];
-#pragma unroll
-        for (int k = 1; k < 8; ++k) x = q == k ? t[k] : x;
-        return x;
-    };
+    const RAOctConst c = kRAOctConsts[q];
     RAOctLane L;
     L.q = q;
     L.lo = q < 4;
     L.vother = q == 5 || q == 6;
-    L.d = pick(d);
-    L.e = lane_div(pick(e));
-    L.g0 = L.vother ? 0.1 : 0.0;
-    L.c = q == 5 ? 0.75 : (q == 6 ? 0.5 : 1.0);
-    L.den = pick(den);
+    L.d = c.d;
+    L.e = c.e;
+    L.g0 = c.g0;
+    L.c = c.c;
+    L.den = MODEL == 1 && q == 7 ? 10.0 : c.den;
     L.dtau = q == 1 || q == 2;
     L.dca = q == 5;
     L.EL = EL;
@@ -425,7 +453,7 @@ __device__ __forceinline__ RAOctLane ra_oct_lane(int q, double EL, double GCa, d
     L.EA = L.lo ? kRA_Egaba : 0.0;
     L.EB = L.lo ? 0.0 : kRA_Egaba;
     L.mu = L.lo ? mu_s : mu_d;
-    L.R = lane_div(L.lo ? 275000.0 : 550000.0);
+    L.R = c.R;
     L.ca01 = -0.1 * GCa;
     L.tab = tab;
     return L;
