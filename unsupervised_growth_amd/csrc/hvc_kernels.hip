@@ -266,11 +266,14 @@ __device__ __forceinline__ void inbox_put(const Inbox& ib, int tgt, int step, in
 
 // The window's clock in LDS: wclk[t - t0 + 1] = clock[t] for t0 - 1 <= t <= t1.
 // First step a >= lo (lo >= t0) with clock[a] >= T (the drain test
-// internal_time >= delivery_time); T <= clock[t1], so a <= t1.
-__device__ __forceinline__ int arrival_step(const double* wclk, int t0, int lo, double T)
+// internal_time >= delivery_time); T <= clock[t1], so a <= t1.  The search
+// starts where T lies at steps of 1 / inv_dt: two LDS reads an edge, where the
+// scan from lo made one, each waiting for the one before, per step.
+__device__ __forceinline__ int arrival_step(const double* wclk, int t0, int t1, int lo, double T, float inv_dt)
 {
-    int a = lo;
+    int a = min(max(lo + (int)((float)(T - wclk[lo - t0]) * inv_dt), lo), t1);
     while (wclk[a - t0 + 1] < T) ++a;
+    while (a > lo && wclk[a - t0] >= T) --a;
     return a;
 }
 
@@ -335,6 +338,7 @@ __device__ __forceinline__ int push_fixed(const NetDev& nd, const double* wclk, 
     FlSlot* more = fl.more + (size_t)pre * (kMaxInflight - kHeadSlots);
     auto slot = [&](int k) -> FlSlot* { return k < kHeadSlots ? &hp->s[k] : more + (k - kHeadSlots); };
     const double tend = wclk[t1 - t0 + 1];
+    const float inv_dt = __builtin_amdgcn_rcpf((float)nd.dt);
     // the held slots and which of them have an edge due in this window
     unsigned held_mask = 0, due_mask = 0;
 #pragma unroll
@@ -413,7 +417,7 @@ __device__ __forceinline__ int push_fixed(const NetDev& nd, const double* wclk, 
             const double dn = d_arr[en];
             const int tgn = tgt_arr[en];
             const double wn = w_arr[en];
-            const int a = arrival_step(wclk, t0, lo, T);
+            const int a = arrival_step(wclk, t0, t1, lo, T, inv_dt);
             lo = a;
             inbox_put(ib, tg, a, pre, w, nd.err);
             cc = cn;
@@ -477,6 +481,11 @@ __device__ __forceinline__ bool stream_peek(const NetDev& nd, int i, int sidx, d
 }
 
 constexpr int kQuadPushNeurons = 65536;   // neurons per context up to which the pushes take a quad per neuron
+// Lanes per neuron of a chain test's RA->RA pushes (no network grows).  One
+// lane wrote a row's ~10-30 records of active edges one atomic after the
+// other, and the role was the last to end in every window that had it.  Where
+// some network grows the role's waves hold one row per lane (rr_row).
+constexpr int kChainPushLanes = 4;
 constexpr int kDeliverRoleWaves = 256;    // waves per role of a delivery launch, at most
 
 // A row's first kRowHeads streams while a window drains them, one column of the
@@ -901,6 +910,7 @@ template <int GA, int GB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_deliver_sweep(NetDev nd, int t0,
                                                                                              int t1, int b0, int b1)
 {
+    kernarg_touch(nd);
     const int b = blockIdx.x, bs = blockDim.x, tid = threadIdx.x;
     __shared__ double wclk[kMaxWindowSteps + 1];
     extern __shared__ double heads_lds[];   // StreamHeads of the block's rows
@@ -940,13 +950,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // this window's integration); the next window's integration fills it
     if (b == 0 && threadIdx.x == 0) *nd.post_list_next_cnt = 0;
     if (b < b0) {
-        // RA->RA: one lane per row
-        const int i = b * blockDim.x + threadIdx.x;
+        // RA->RA: one lane per row (kChainPushLanes in a chain test)
+        const int G0 = nd.growth_mode == 0 ? kChainPushLanes : 1;
+        const int i = (b * bs + tid) / G0;
         if (i >= nd.n_ra) return;
         const StreamHeads hd{heads_lds + tid, (int*)(heads_lds + kHeadDoubles * kRowHeads * bs) + tid, bs};
         const int growth = nd.growth_mode == 2 ? nd.net_growth[nd.ra_net[i]] : nd.growth_mode;
         if (growth)
             rr_row(nd, wclk, i, t0, t1, hd);
+        else if (nd.growth_mode == 0)
+            push_fixed<kChainPushLanes>(nd, wclk, i, tid % kChainPushLanes, nd.rr_ptr[i], nd.rr_ptr[i] + nd.act_cnt[i],
+                                        nd.chain_e, nd.rr_tgt, nd.w, nd.rr_d, nd.fl_rr, nd.fl_rr.head[i],
+                                        nd.soma_mask[i], t0, t1, nd.in_ge_ra);
         else
             push_fixed<1>(nd, wclk, i, 0, nd.rr_ptr[i], nd.rr_ptr[i] + nd.act_cnt[i], nd.chain_e, nd.rr_tgt, nd.w,
                           nd.rr_d, nd.fl_rr, nd.fl_rr.head[i], nd.soma_mask[i], t0, t1, nd.in_ge_ra);
@@ -967,17 +982,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // the previous window (listed here), so it reads the rows, slot tables and
 // edges of its active neurons and nothing else.  Item k of a role goes to wave
 // k mod W (W = the role's waves): up to W items run one per wave, side by side.
+// A launch is a chain of memory latencies (arguments; clock, count and item;
+// the item's state; its edges; the records' atomics), not work: kernarg_touch
+// reads the arguments in one round where each branch waited for its own.
+// With the search of arrival_step and kChainPushLanes, per window (timing
+// events included, ~2.7 us of it): chain test 1 000 + 280 neurons 11.6 -> 8.5
+// us, growth 300 + 30 11.0 -> 9.6, 5 003 + 1 377 13.6 -> 11.4, FP32 pool of 4
+// 14.5 -> 11.9; sweep form, 20 000 + 5 500 10.8 -> 10.3.  More lanes for the
+// fixed-weight pushes (RA->I 4 or 16, I->RA 16, 32 or 64) gained nothing: few
+// edges of a spike are due in one window.
 // ---------------------------------------------------------------------------
 template <int GA, int GB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_deliver_list(NetDev nd, int t0,
                                                                                             int t1, int b0, int b1)
 {
+    kernarg_touch(nd);
     const int b = blockIdx.x, bs = blockDim.x, tid = threadIdx.x;
     const int w = nd.window;
     __shared__ double wclk[kMaxWindowSteps + 1];
     extern __shared__ double heads_lds[];   // StreamHeads of the block's rows
     const int role = b < b0 ? 0 : (b < b0 + b1 ? 1 : 2);
-    const int G = role == 0 ? 1 : (role == 1 ? GA : GB);
+    const int G = role == 0 ? (nd.growth_mode == 0 ? kChainPushLanes : 1) : (role == 1 ? GA : GB);
     const int wpb = bs >> 6;
     const int nwaves = (role == 0 ? b0 : (role == 1 ? b1 : (int)gridDim.x - b0 - b1)) * wpb;
     const int wave = (b - (role == 0 ? 0 : (role == 1 ? b0 : b0 + b1))) * wpb + (tid >> 6);
@@ -1013,6 +1038,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             const int growth = nd.growth_mode == 2 ? nd.net_growth[nd.ra_net[i]] : nd.growth_mode;
             if (growth)
                 left = rr_row(nd, wclk, i, t0, t1, hd);
+            else if (nd.growth_mode == 0)
+                left = push_fixed<kChainPushLanes>(nd, wclk, i, r, nd.rr_ptr[i], nd.rr_ptr[i] + nd.act_cnt[i],
+                                                   nd.chain_e, nd.rr_tgt, nd.w, nd.rr_d, nd.fl_rr, nd.fl_rr.head[i],
+                                                   nd.soma_mask[i], t0, t1, nd.in_ge_ra);
             else
                 left = push_fixed<1>(nd, wclk, i, 0, nd.rr_ptr[i], nd.rr_ptr[i] + nd.act_cnt[i], nd.chain_e,
                                      nd.rr_tgt, nd.w, nd.rr_d, nd.fl_rr, nd.fl_rr.head[i], nd.soma_mask[i], t0, t1,
@@ -1163,15 +1192,16 @@ void launch_deliver(hipStream_t st, const NetDev& nd, int t0, int t1, const Tuni
     // size; the sweep's grid grows with the neurons, and above
     // kQuadPushNeurons its extra waves cost more than they save, so every
     // push takes one lane there.
+    const long long rows = (nd.growth_mode == 0 ? kChainPushLanes : 1ll) * nd.n_ra;
     if (tu.deliver_lists || nd.n_ra + nd.n_i <= kQuadPushNeurons) {
-        const int b0 = role_blocks(nd.n_ra), b1 = role_blocks(nd.n_ra), b2 = role_blocks(4ll * nd.n_i);
+        const int b0 = role_blocks(rows), b1 = role_blocks(nd.n_ra), b2 = role_blocks(4ll * nd.n_i);
         if (b0 + b1 + b2 == 0) return;
         if (tu.deliver_lists)
             k_deliver_list<1, 4><<<b0 + b1 + b2, bs, lds, st>>>(nd, t0, t1, b0, b1);
         else
             k_deliver_sweep<1, 4><<<b0 + b1 + b2, bs, lds, st>>>(nd, t0, t1, b0, b1);
     } else {
-        const int b0 = role_blocks(nd.n_ra), b1 = role_blocks(nd.n_ra), b2 = role_blocks(nd.n_i);
+        const int b0 = role_blocks(rows), b1 = role_blocks(nd.n_ra), b2 = role_blocks(nd.n_i);
         if (b0 + b1 + b2 == 0) return;
         k_deliver_sweep<1, 1><<<b0 + b1 + b2, bs, lds, st>>>(nd, t0, t1, b0, b1);
     }
