@@ -1098,22 +1098,40 @@ __global__ __launch_bounds__(512) void k_sync(NetDev nd)
     }
 }
 
-// end of a growth trial: potentiation_decay + update_all_synapses (NGS:9567-9570)
+// end of a growth trial: potentiation_decay + update_all_synapses
+// (NGS:9567-9570), one wave per row.  The decay is a stream over the edges
+// (17 bytes read and 8 written each), 64 at a time; update_synapse changes
+// nothing for an edge whose flags already agree with its weight, so only the
+// others take it, in the row's order, on the wave's first lane.  One thread
+// per row read a cache line per edge and array: 1 700 us at 2 000 rows of
+// 1 999 edges, now 29 us (100 MB, 3.4 TB/s); 280 -> 7 us at 300 dense rows.
 __global__ __launch_bounds__(256) void k_decay(NetDev nd)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = __lane_id();
     if (i >= nd.n_ra || !nd.net_growth[nd.ra_net[i]]) return;
     const hvc_synaptic_params& p = nd.syn;
-    for (int e = nd.rr_ptr[i]; e < nd.rr_ptr[i + 1]; ++e) {
-        double w = nd.w[e];
-        if (w >= p.SUPERSYNAPSE_THRESHOLD)
-            w -= p.BETA_SUPERSYNAPSE;
-        else
-            w -= p.BETA;
-        if (w < 0) w = 0;
-        nd.w[e] = w;
+    const int end = nd.rr_ptr[i + 1];
+    for (int e0 = nd.rr_ptr[i]; e0 < end; e0 += 64) {
+        const int e = e0 + lane;
+        bool differs = false;
+        if (e < end) {
+            double w = nd.w[e];
+            const int act = nd.act[e], sup = nd.sup[e];
+            if (w >= p.SUPERSYNAPSE_THRESHOLD)
+                w -= p.BETA_SUPERSYNAPSE;
+            else
+                w -= p.BETA;
+            if (w < 0) w = 0;
+            nd.w[e] = w;
+            // (the conditions of update_synapse on the edge alone)
+            differs = (w >= p.ACTIVATION_THRESHOLD && act == 0) || (w >= p.SUPERSYNAPSE_THRESHOLD && sup == 0) ||
+                      (w < p.SUPERSYNAPSE_THRESHOLD && sup == 1) || (w < p.ACTIVATION_THRESHOLD && act == 1);
+        }
+        uint64_t m = __ballot(differs);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // lane 0 reads the other lanes' weights
+        if (lane == 0)
+            for (; m; m &= m - 1) update_synapse(nd, i, e0 + __ffsll((unsigned long long)m) - 1);
     }
-    update_row(nd, i);
 }
 
 // chain test: each row's active edges sorted by (delay, target)
@@ -1261,7 +1279,7 @@ void launch_sync(hipStream_t st, const NetDev& nd, const Tuning& tu)
 
 void launch_decay(hipStream_t st, const NetDev& nd)
 {
-    k_decay<<<blocks_for(nd.n_ra, 64), 64, 0, st>>>(nd);
+    k_decay<<<blocks_for(nd.n_ra, 4), 256, 0, st>>>(nd);
 }
 
 void launch_eval_math(hipStream_t st, int fn, int n, const double* a, const double* b, double* out)
