@@ -161,12 +161,14 @@ hvc_status hvc_batch_download_synapses(hvc_ctx* ctx, int net, hvc_synapses* syn)
 hvc_status hvc_batch_upload_synapses(hvc_ctx* ctx, int net, const hvc_synapses* syn);
 
 /* Launch shapes of the per-window kernels.  hvc_autotune times the candidates
- * on the resident networks (a scratch chain test through the first `windows`
- * coupling windows, kicked early so that activity propagates; synapse state is
- * not touched and the next trial starts from rest as always), keeps the fastest
- * and returns it with its per-window device times (ms) of integrate, deliver
- * and sync.  Results do not depend on the launch shapes.  No counterpart in the
- * reference. */
+ * on the resident networks (a scratch trial through the first `windows` coupling
+ * windows, launched as a growth trial's windows or, in a serving pool, a chain
+ * test's, kicked early so that activity propagates; synapse state is not touched
+ * and the next trial starts from rest as always), integration and delivery
+ * shapes in pairs by the time of whole windows, keeps the fastest pair and
+ * returns it with its device times (ms) of integrate and deliver per window and
+ * of one sync.  Results do not depend on the launch shapes.  No counterpart in
+ * the reference. */
 typedef struct {
     int integrate_block;   /* threads per block of the integration kernel: 64, 128, 256 */
     int i_lanes;           /* HVC-I DP8: 3 = eight lanes per neuron, 2 = four lanes, 1 = five lanes,

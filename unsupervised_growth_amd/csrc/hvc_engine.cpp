@@ -1396,11 +1396,17 @@ extern "C" hvc_status hvc_set_tuning(hvc_ctx* ctx, const hvc_tuning* t)
     return HVC_OK;
 }
 
-// A scratch chain test of every resident network (synapse state untouched, the
-// training kick 5 ms after the start so that chains are active) through the
-// first `windows` coupling windows; average device time per window of each
-// kernel class under tuning tu.
-static hvc_status timed_windows(hvc_ctx* ctx, int windows, const Tuning& tu, double ms[3])
+// A scratch trial of every resident network (synapse state untouched, the
+// training kick 5 ms after the start so that spikes propagate) through the first
+// `windows` coupling windows under tuning tu, launched as run_impl launches them:
+// integration and delivery back to back, and with grow the growth trial's
+// delivery roles and STDP blocks.  No network is marked as growing, so no
+// postsynaptic event arises and neither the deliveries nor the STDP blocks find
+// a weight to change.  window_ms: device time per window, the windows as a
+// whole.  kernel_ms (or nullptr): integrate, deliver and sync on their own, with
+// an event after every launch, which the windows of a trial do not have.
+static hvc_status timed_windows(hvc_ctx* ctx, int windows, const Tuning& tu, bool grow, double& window_ms,
+                                double* kernel_ms)
 {
     NetDev& nd = ctx->nd;
     hipStream_t s = ctx->stream;
@@ -1421,45 +1427,54 @@ static hvc_status timed_windows(hvc_ctx* ctx, int windows, const Tuning& tu, dou
     HVC_TRY(hipMemcpyAsync(ctx->d_net_first, zeros.data(), sizeof(int) * B, hipMemcpyHostToDevice, s));
     HVC_TRY(hipMemcpyAsync(ctx->d_net_trial, trial.data(), sizeof(uint32_t) * B, hipMemcpyHostToDevice, s));
     refresh_rr_pos(ctx, nd);
-    nd.growth_mode = 0;   // chain tests only
+    nd.growth_mode = grow ? 1 : 0;
     nd.net_live = nullptr;
     launch_reset(s, nd, ctx->E);
-    launch_chain_edges(s, nd);
+    if (!grow) launch_chain_edges(s, nd);
+    constexpr int kSyncs = 4;
     const int nw = std::min(windows, (int)ctx->windows.size());
     CallEvents events;
-    HVC_TRY(events.create(6 * (size_t)nw));
+    HVC_TRY(events.create(kernel_ms ? 2 * (size_t)nw + 2 : 2));
     std::vector<hipEvent_t>& ev = events.ev;
     hvc_status r = HVC_OK;
+    hipEventRecord(ev[0], s);
     for (int w = 0; w < nw; ++w) {
         int t0 = ctx->windows[w].first, t1 = ctx->windows[w].second;
         noise_chunk(ctx, nd, w);
-        hipEventRecord(ev[6 * w + 0], s);
-        const StdpArgs none{nd.post_list, nd.post_list_cnt, 0};
+        const StdpArgs sa{nd.post_list, nd.post_list_cnt, w > 0 ? ctx->windows[w - 1].second : 0};
+        const int stdp = grow && w > 0;
         NetDev nv = nd;
         nv.window = w;
         nv.wl_on = tu.deliver_lists;
+        if (kernel_ms) hipEventRecord(ev[2 * w], s);
         if (ctx->prm.precision == 1)
-            launch_integrate_f32(s, nv, t0, t1, tu, none, 0);
+            launch_integrate_f32(s, nv, t0, t1, tu, sa, stdp);
         else
-            launch_integrate(s, nv, t0, t1, tu, none, 0);
-        hipEventRecord(ev[6 * w + 1], s);
+            launch_integrate(s, nv, t0, t1, tu, sa, stdp);
+        if (kernel_ms) hipEventRecord(ev[2 * w + 1], s);
         launch_deliver(s, nv, t0, t1, tu);
-        hipEventRecord(ev[6 * w + 2], s);
-        hipEventRecord(ev[6 * w + 3], s);
-        launch_sync(s, nd, tu);
-        hipEventRecord(ev[6 * w + 4], s);
+    }
+    hipEventRecord(ev[kernel_ms ? 2 * nw : 1], s);
+    if (kernel_ms) {
+        for (int k = 0; k < kSyncs; ++k) launch_sync(s, nd, tu);
+        hipEventRecord(ev[2 * nw + 1], s);
     }
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess) r = fail(ctx, HVC_E_HIP, std::string("autotune: ") + hipGetErrorString(e));
-    ms[0] = ms[1] = ms[2] = 0;
-    for (int w = 0; w < nw && r == HVC_OK; ++w) {
-        float a = 0, b = 0, c = 0;
-        hipEventElapsedTime(&a, ev[6 * w + 0], ev[6 * w + 1]);
-        hipEventElapsedTime(&b, ev[6 * w + 1], ev[6 * w + 2]);
-        hipEventElapsedTime(&c, ev[6 * w + 3], ev[6 * w + 4]);
-        ms[0] += a; ms[1] += b; ms[2] += c;
+    auto between = [&](int a, int b) {
+        float ms = 0;
+        hipEventElapsedTime(&ms, ev[a], ev[b]);
+        return (double)ms;
+    };
+    if (r == HVC_OK) window_ms = between(0, kernel_ms ? 2 * nw : 1) / std::max(nw, 1);
+    if (kernel_ms && r == HVC_OK) {
+        kernel_ms[0] = kernel_ms[1] = 0;
+        for (int w = 0; w < nw; ++w) {
+            kernel_ms[0] += between(2 * w, 2 * w + 1) / nw;
+            kernel_ms[1] += between(2 * w + 1, 2 * w + 2) / nw;
+        }
+        kernel_ms[2] = between(2 * nw, 2 * nw + 1) / kSyncs;
     }
-    for (int k = 0; k < 3; ++k) ms[k] /= std::max(nw, 1);
     unsigned int err = 0;
     HVC_TRY(hipMemcpy(&err, nd.err, sizeof(err), hipMemcpyDeviceToHost));
     if (err && r == HVC_OK) r = fail(ctx, HVC_E_CAPACITY, "autotune: engine capacity exceeded in the scratch run");
@@ -1467,20 +1482,47 @@ static hvc_status timed_windows(hvc_ctx* ctx, int windows, const Tuning& tu, dou
     return r;
 }
 
+// The shapes of integration and delivery are chosen as pairs, by the time of
+// whole windows: with one-wave blocks the SIMDs that an integration's waves land
+// on depend on the delivery launched before it.  (20 000 + 5 500 neurons, FP32
+// growth trial: k_integrate 23.6 us in blocks of 64 after deliveries in blocks
+// of 64 or 256, 29.7 us after blocks of 128; in blocks of 256 23.4 us after all
+// three.  Chosen one after the other, each under the other's default, the two
+// came out as 64 and 128: 71.3 ms per trial, 58.9 ms as a pair.)  The
+// integration shapes are timed under the present delivery shape, the best of
+// them under every delivery shape, and the best pairs again.
 extern "C" hvc_status hvc_autotune(hvc_ctx* ctx, int windows, hvc_tuning* best, double* ms_out)
 {
     if (!ctx || windows <= 0) return HVC_E_ARG;
     ApiLock lk(ctx);   // between a pool's serving rounds
     if (!ctx->uploaded || ctx->n_nets == 0) return fail(ctx, HVC_E_STATE, "upload networks first");
     HVC_TRY(hipSetDevice(ctx->device));
-    Tuning tu = ctx->tuning;
-    double ms[3], best_ms[3];
+    const Tuning tu = ctx->tuning;
+    bool grow = !ctx->pool;   // a pool serves chain tests
     hvc_status r;
+    auto timed = [&](const Tuning& t, int n, double& ms, double* kernel_ms) {
+        hvc_status q = timed_windows(ctx, n, t, grow, ms, kernel_ms);
+        if (q == HVC_E_CAPACITY && grow) {   // (a growing network's streams may overflow where its chain test runs)
+            grow = false;
+            q = timed_windows(ctx, n, t, grow, ms, kernel_ms);
+        }
+        return q;
+    };
+    struct Candidate {
+        Tuning tu;
+        double ms;
+    };
+    std::vector<Candidate> cand;
+    auto add = [&](const Tuning& t) {
+        cand.push_back({t, 0.0});
+        return timed(t, windows, cand.back().ms, nullptr);
+    };
+    auto sort = [&] {
+        std::stable_sort(cand.begin(), cand.end(), [](const Candidate& a, const Candidate& b) { return a.ms < b.ms; });
+    };
     // integrate: block size and the HVC-I and HVC-RA layouts (four, five and
     // eight lanes per HVC-I neuron exist for DP8 only, FP32's four per HVC-RA
     // neuron for RK4 only; in FP64 every layout with several lanes is eight)
-    double bi = 1e30;
-    Tuning ti = tu;
     const bool f64 = ctx->prm.precision == 0;
     for (int ra_lanes = (ctx->prm.ra_model == 1 || f64 ? 1 : 0); ra_lanes >= 0; --ra_lanes)
         for (int lanes = (ctx->prm.i_model == 0 ? 3 : 0); lanes >= 0; --lanes) {
@@ -1490,35 +1532,42 @@ extern "C" hvc_status hvc_autotune(hvc_ctx* ctx, int windows, hvc_tuning* best, 
                 c.integrate_block = bs;
                 c.i_lanes = lanes;
                 c.ra_lanes = ra_lanes;
-                if ((r = timed_windows(ctx, windows, c, ms)) != HVC_OK) return r;
-                if (ms[0] < bi) { bi = ms[0]; ti = c; }
+                if ((r = add(c)) != HVC_OK) return r;
             }
         }
-    tu = ti;
-    double bd = 1e30;
-    Tuning td = tu;
-    for (int lists = 1; lists >= 0; --lists)
-        for (int bs : {64, 128, 256}) {
-            Tuning c = tu;
-            c.deliver_block = bs;
-            c.deliver_lists = lists;
-            if ((r = timed_windows(ctx, windows, c, ms)) != HVC_OK) return r;
-            if (ms[1] < bd) { bd = ms[1]; td = c; }
+    constexpr size_t kKept = 4;   // integration shapes paired with every delivery shape; pairs timed again
+    sort();
+    const std::vector<Candidate> shapes(cand.begin(), cand.begin() + std::min(kKept, cand.size()));
+    for (const Candidate& s : shapes)
+        for (int lists = 1; lists >= 0; --lists)
+            for (int bs : {64, 128, 256}) {
+                if (bs == tu.deliver_block && lists == tu.deliver_lists) continue;
+                Tuning c = s.tu;
+                c.deliver_block = bs;
+                c.deliver_lists = lists;
+                if ((r = add(c)) != HVC_OK) return r;
+            }
+    sort();
+    cand.resize(std::min(kKept, cand.size()));
+    for (int again = 0; again < 2; ++again)
+        for (Candidate& c : cand) {
+            double ms = 0;
+            if ((r = timed(c.tu, windows, ms, nullptr)) != HVC_OK) return r;
+            c.ms = std::min(c.ms, ms);
         }
-    tu = td;
-    double bsy = 1e30;
-    Tuning ts = tu;
+    sort();
+    Tuning ts = cand[0].tu;
+    double ms, kernel_ms[3], bsy = 1e30;
     for (int bs : {128, 256, 512}) {
-        Tuning c = tu;
+        Tuning c = cand[0].tu;
         c.sync_block = bs;
-        if ((r = timed_windows(ctx, windows, c, ms)) != HVC_OK) return r;
-        if (ms[2] < bsy) { bsy = ms[2]; ts = c; }
+        if ((r = timed(c, std::min(windows, 32), ms, kernel_ms)) != HVC_OK) return r;
+        if (kernel_ms[2] < bsy) { bsy = kernel_ms[2]; ts = c; }
     }
-    tu = ts;
-    if ((r = timed_windows(ctx, windows, tu, best_ms)) != HVC_OK) return r;
-    ctx->tuning = tu;
+    if ((r = timed(ts, windows, ms, kernel_ms)) != HVC_OK) return r;
+    ctx->tuning = ts;
     if (best) hvc_get_tuning(ctx, best);
-    if (ms_out) for (int k = 0; k < 3; ++k) ms_out[k] = best_ms[k];
+    if (ms_out) for (int k = 0; k < 3; ++k) ms_out[k] = kernel_ms[k];
     return HVC_OK;
 }
 
