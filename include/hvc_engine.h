@@ -176,8 +176,9 @@ typedef struct {
     int deliver_block;     /* 64, 128, 256 */
     int sync_block;        /* 64 .. 512 */
     int ra_lanes;          /* FP32 form, HVC-RA RK4: 1 = four lanes per neuron, 0 = one thread per neuron.
-                              FP64 form, both HVC-RA models: 1 = eight lanes per neuron, 0 = eight lanes for
-                              networks small enough to gain by it, else one thread */
+                              FP64 form, both HVC-RA models: 1 = eight lanes per neuron (RK4: four in
+                              networks large enough to gain by it), 0 = eight lanes for networks small
+                              enough to gain by it, else one thread */
     int deliver_lists;     /* 1 = the delivery visits only the neurons that spiked in the window or
                               still have spikes in flight (lists kept on the device), 0 = it reads
                               every neuron's queue state each window */

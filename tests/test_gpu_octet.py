@@ -1,7 +1,7 @@
 """The FP64 octet steppers (eight lanes per neuron) where they can go wrong, bit
 for bit against the oracle: partly filled waves, steps that leave the range of
-the fast quotients and repeat with IEEE division, and a network too large for
-octets, which takes one thread per neuron."""
+the fast quotients and repeat with IEEE division, and networks too large for
+octets, which take four lanes or one thread per neuron."""
 import dataclasses
 
 import numpy as np
@@ -75,22 +75,58 @@ def test_steps_out_of_the_fast_range(model):
     assert r.bad_values == -1 and not np.isfinite(r.i_state).all() and (abs(r.ra_state[:4, 0]) > 2000).any()
 
 
-@pytest.mark.parametrize("model,n_ra", [(0, 32769), (1, 16385)])
-def test_large_network_takes_one_thread_per_neuron(model, n_ra):
-    from unsupervised_growth_amd.network import random_network
-    small = random_network(5, 3, n_train=2, p_ra2i=0.5, p_i2ra=0.5, seed=4, rr=2)
-    pad = n_ra - 5
+def _padded(small, n_ra):
+    """The network with n_ra - small.n_ra unconnected HVC-RA neurons after its own."""
+    pad = n_ra - small.n_ra
 
     def more(ptr):
         return np.concatenate([ptr, np.full(pad, ptr[-1], np.int32)])
 
     z = np.zeros(pad, np.int32)
-    net = dataclasses.replace(small, n_ra=n_ra, ra2i_ptr=more(small.ra2i_ptr), rr_ptr=more(small.rr_ptr),
-                              act_cnt=np.concatenate([small.act_cnt, z]), sup_cnt=np.concatenate([small.sup_cnt, z]),
-                              remodeled=np.concatenate([small.remodeled, z]),
-                              erest=np.concatenate([small.erest, np.linspace(-90.0, -60.0, pad)]),
-                              gca=np.concatenate([small.gca, np.linspace(0.0, 60.0, pad)]))
-    _compare(net, 3.0, ra_model=model)
+    return dataclasses.replace(small, n_ra=n_ra, ra2i_ptr=more(small.ra2i_ptr), rr_ptr=more(small.rr_ptr),
+                               act_cnt=np.concatenate([small.act_cnt, z]), sup_cnt=np.concatenate([small.sup_cnt, z]),
+                               remodeled=np.concatenate([small.remodeled, z]),
+                               erest=np.concatenate([small.erest, np.linspace(-90.0, -60.0, pad)]),
+                               gca=np.concatenate([small.gca, np.linspace(0.0, 60.0, pad)]))
+
+
+@pytest.mark.parametrize("model,n_ra", [(0, 32769), (1, 16385)])
+def test_large_network_takes_one_thread_per_neuron(model, n_ra):
+    from unsupervised_growth_amd.network import random_network
+    small = random_network(5, 3, n_train=2, p_ra2i=0.5, p_i2ra=0.5, seed=4, rr=2)
+    _compare(_padded(small, n_ra), 3.0, ra_model=model)
+
+
+@pytest.mark.parametrize("model,n_ra,ra_lanes", [(1, 14337, 1)])
+def test_large_network_through_a_kick(model, n_ra, ra_lanes):
+    """The layouts of large networks (four lanes in the RK4 model) with their
+    spikes, deliveries and STDP: two trials kicked at their start."""
+    from unsupervised_growth_amd.engine import Engine
+    from unsupervised_growth_amd.network import random_network
+    small = random_network(20, 6, n_train=8, p_ra2i=0.5, p_i2ra=0.5, seed=4, w_rr=150.0, delays=("uniform", 0.0, 2.0),
+                           rr_delays=("uniform", 0.0, 2.0))
+    net = _padded(small, n_ra)
+    kw = dict(ra_model=model, ra_poisson=model, trial_ms=9.0)
+    ora = OracleSim(net, **kw)
+    with Engine(**kw) as eng:
+        eng.upload(net)
+        eng.set_tuning(ra_lanes=ra_lanes)
+        for k in range(2):
+            tr = dict(mode=0, trial_index=k, first_trial=k == 0, mean_injection_time=0.5)
+            o, r = ora.run_trial(**tr), eng.run_trial(want_state=True, **tr)
+            for kind in ("soma", "dend", "interneuron"):
+                for a, b in zip(getattr(r, kind), o[kind]):
+                    np.testing.assert_array_equal(a, b)
+            np.testing.assert_array_equal(r.ra_state, o["ra_state"])
+            np.testing.assert_array_equal(r.i_state, o["i_state"])
+            s, want = eng.download_synapses(), ora.synapses()
+            for f in ("w", "act_cnt", "act_ids", "sup_cnt", "sup_ids", "remodeled"):
+                np.testing.assert_array_equal(getattr(s, f), want[f], err_msg=f)
+            for kind in ("soma", "dend", "interneuron"):
+                assert sum(map(len, getattr(r, kind)[:20])) > 0, kind
+            assert (s.w != small.rr_w).all() and s.act_cnt.any()
+            # inhibition and, once synapses are active, excitation has reached the neurons
+            assert (r.ra_state[:20, 11] > 0).any() and (r.i_state[:, 5] > 0).any()
 
 
 @pytest.mark.parametrize("model,poisson", [(0, 0), (1, 1)])

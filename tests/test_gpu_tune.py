@@ -1,5 +1,5 @@
 """The autotuner: the shape it keeps is a pair that is fast together, and its
-scratch trials leave the networks as they were."""
+scratch trials leave the networks as they were; and a layout that it has to find."""
 import time
 
 import numpy as np
@@ -66,3 +66,25 @@ def test_scratch_trials_leave_the_network(precision):
             for x, y in zip(getattr(a, kind), getattr(b, kind)):
                 np.testing.assert_array_equal(x, y)
     assert sum(map(len, runs[0][0][1].soma)) > 0
+
+
+def test_fp64_rk4_has_a_layout_between_octets_and_one_thread():
+    """At 20 000 HVC-RA neurons four lanes per neuron take 61 us per window of
+    k_integrate where eight take 76 and one thread 79."""
+    from unsupervised_growth_amd import configs
+    from unsupervised_growth_amd.engine import Engine
+    net, kw = configs.c3()
+    us = {}
+    with Engine(ra_model=1, precision=0, **dict(kw, trial_ms=40.0)) as eng:
+        eng.upload(net)
+        eng.set_timing(True)
+        for lanes in (1, 0):
+            eng.set_tuning(ra_lanes=lanes)
+            took = []
+            for k in range(3):
+                eng.set_timing(True)
+                eng.run_trial(mode=0, training=True, trial_index=k, first_trial=k == 0, mean_injection_time=10.0)
+                took.append(1000.0 * eng.kernel_timing("integrate")[0])
+            us[lanes] = min(took)
+    print("k_integrate us per window", us, flush=True)
+    assert us[1] < 0.9 * us[0]

@@ -34,6 +34,7 @@ void launch_trace_ra(hipStream_t st, const NetDev& nd, int n, int n_steps, uint3
 void launch_trace_i(hipStream_t st, const NetDev& nd, int n, int n_steps, int first_trial, uint32_t trial,
                     const double* exc_g, const double* inh_g, double* out, uint8_t* fired);
 void launch_reset(hipStream_t st, const NetDev& nd, int E);
+int ra_lanes_f64(int ra_model, int n_ra, int ra_lanes);   // lanes per HVC-RA neuron: 8, 4 or 1
 void launch_integrate(hipStream_t st, const NetDev& nd, int t0, int t1, const Tuning& tu, const StdpArgs& sa,
                       int stdp);
 void launch_trace_ra_f32(hipStream_t st, const NetDev& nd, int n, int n_steps, uint32_t trial, const double* EL,
@@ -1521,10 +1522,12 @@ extern "C" hvc_status hvc_autotune(hvc_ctx* ctx, int windows, hvc_tuning* best, 
         std::stable_sort(cand.begin(), cand.end(), [](const Candidate& a, const Candidate& b) { return a.ms < b.ms; });
     };
     // integrate: block size and the HVC-I and HVC-RA layouts (four, five and
-    // eight lanes per HVC-I neuron exist for DP8 only, FP32's four per HVC-RA
-    // neuron for RK4 only; in FP64 every layout with several lanes is eight)
+    // eight lanes per HVC-I neuron exist for DP8 only, in FP64 all of them eight;
+    // FP32's four per HVC-RA neuron for RK4 only, FP64's values may mean the same)
     const bool f64 = ctx->prm.precision == 0;
-    for (int ra_lanes = (ctx->prm.ra_model == 1 || f64 ? 1 : 0); ra_lanes >= 0; --ra_lanes)
+    auto f64_lanes = [&](int ra_lanes) { return ra_lanes_f64(ctx->prm.ra_model, ctx->n_ra, ra_lanes); };
+    const bool several = f64 ? f64_lanes(1) != f64_lanes(0) : ctx->prm.ra_model == 1;
+    for (int ra_lanes = several ? 1 : 0; ra_lanes >= 0; --ra_lanes)
         for (int lanes = (ctx->prm.i_model == 0 ? 3 : 0); lanes >= 0; --lanes) {
             if (f64 && (lanes == 1 || lanes == 2)) continue;
             for (int bs : {64, 128, 256}) {

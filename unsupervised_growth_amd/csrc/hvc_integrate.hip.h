@@ -80,9 +80,9 @@ __device__ __forceinline__ void ra_step_debraband(RAState& s, real el, real gca,
                      (ra_debraband<true>(bad, s, el, gca, u, J1s, J2s, J1d, J2d, E_dt, E_half)))
 }
 
-template <bool LANES = false, class Slot = int>
+template <bool LANES = false>
 __device__ __forceinline__ void ra_step_runge4(RAState& s, real el, real gca, const RAUniform& u, real E_third,
-                                               real E_twothird, real E_dt, const Slot* sl = nullptr)
+                                               real E_twothird, real E_dt, const RAGateSlot* sl = nullptr)
 {
     HVC_GUARDED_STEP(RAState, (ra_runge4<false, LANES>(bad, s, el, gca, u, sl, E_third, E_twothird, E_dt)),
                      (ra_runge4<true, LANES>(bad, s, el, gca, u, sl, E_third, E_twothird, E_dt)))
@@ -395,7 +395,7 @@ __device__ __forceinline__ int ra_window_logs(const NetDev& nd, const Win& win, 
 }
 
 // HVC-RA neurons: one thread per neuron (LANES false, `slot` = neuron index) or,
-// RK4 model in the FP32 form, four lanes per neuron (LANES true, `slot` = wave index; the quad's
+// RK4 model, four lanes per neuron (LANES true, `slot` = wave index; the quad's
 // first lane does the neuron's logging and stores)
 template <int MODEL, bool LANES>
 __device__ void integrate_ra(const NetDev& nd, const Win& win, int slot, int t0, int t1)
@@ -404,16 +404,11 @@ __device__ void integrate_ra(const NetDev& nd, const Win& win, int slot, int t0,
     const int lane = LANES ? __lane_id() : 0;
     const int i = LANES ? slot * kRANeuronsPerWave + (lane >> 2) : slot;
     const bool leader = !LANES || (lane & 3) == 0;
-#ifdef HVC_FP32
     RAGateSlot gs[2];
     if (LANES) {
         gs[0] = kRAGates[2 * (lane & 3)];
         gs[1] = kRAGates[2 * (lane & 3) + 1];
     }
-#else
-    static_assert(!LANES, "four lanes per neuron: FP32 form");
-    const int* gs = nullptr;
-#endif
     const bool live = i < nd.n_ra && (!nd.net_live || nd.net_live[nd.ra_net[i]]);
     const int ii = live ? i : 0;
     const int growth = nd.net_growth[nd.ra_net[ii]];
@@ -971,10 +966,9 @@ __device__ __forceinline__ void kernarg_touch(const NetDev& nd)
 // (one row per thread, sa).
 // LANES: HVC-I bit 0 = five lanes, bit 2 = four lanes, bit 3 = eight lanes per
 // neuron, bit 4 = eight lanes with the one-thread arithmetic (FP32 form), none
-// = one thread; HVC-RA bit 1 = four lanes (FP32 form) or eight
-// (FP64 form), else one thread.  (The layouts are template parameters: a
-// kernel holds the register allocation of one layout only.  The FP64 form has
-// the octets and one thread.)
+// = one thread; HVC-RA bit 1 = four lanes (FP32 form) or eight (FP64 form),
+// bit 5 = four lanes (FP64 form), else one thread.  (The layouts are template
+// parameters: a kernel holds the register allocation of one layout only.)
 template <int RA_MODEL, int I_MODEL, int LANES>
 __global__ __launch_bounds__(256) void k_integrate(NetDev nd, int t0, int t1, int iblocks, int rblocks, StdpArgs sa)
 {
@@ -1023,6 +1017,8 @@ __global__ __launch_bounds__(256) void k_integrate(NetDev nd, int t0, int t1, in
     } else {
         if constexpr ((LANES & 2) != 0)
             integrate_ra_oct<RA_MODEL>(nd, win, lds, rwave, t0, t1);
+        else if constexpr ((LANES & 32) != 0)
+            integrate_ra<RA_MODEL, true>(nd, win, rwave, t0, t1);
         else
             integrate_ra<RA_MODEL, false>(nd, win, (blockIdx.x - iblocks) * blockDim.x + threadIdx.x, t0, t1);
     }
@@ -1345,6 +1341,19 @@ constexpr int kIOctSharedMaxNeurons = 10240;
 // 20 000 neurons, 106 / 116 at 30 000, 134 / 117 at 40 000; RK4 76 / 82 at
 // 20 000, 99 / 99 at 30 000, 126 / 99 at 40 000.
 constexpr int kRAOctMaxNeurons[2] = {32768, 16384};   // by ra_model
+// HVC-RA neurons up to which "several lanes" is eight in the RK4 model, above
+// which it is four: half the waves, so two to a SIMD hold out to 21 000 neurons
+// instead of 13 000.  k_integrate per window beside HVC-I octets, four lanes /
+// eight / one thread, us: 59 / 49 / 77 at 12 000 neurons, 60 / 57 / 77 at
+// 14 000, 60 / 71 / 77 at 16 000, 61 / 76 / 79 at 20 000, 87 / 82 / 98 at
+// 22 000, 88 / 99 / 98 at 28 000, 111 / 110 / 98 at 32 000.
+constexpr int kRAOctMaxOverQuads = 14336;
+
+int ra_lanes_f64(int ra_model, int n_ra, int ra_lanes)
+{
+    if (ra_model == 1 && ra_lanes) return n_ra <= kRAOctMaxOverQuads ? 8 : 4;
+    return ra_lanes || n_ra <= kRAOctMaxNeurons[ra_model == 1] ? 8 : 1;
+}
 // HVC-I neurons up to which a trace takes octets (a trace has no launch shape):
 // beside one-thread HVC-RA waves k_integrate takes 149 us per window with
 // octets, 204 with one thread at 16 500 HVC-I neurons, 224 / 206 at 24 750
@@ -1407,11 +1416,10 @@ void HVC_LAUNCHER(launch_integrate)(hipStream_t st, const NetDev& nd, int t0, in
 #else
     // the FP64 layouts give the same bits, so every HVC-I layout with several
     // lanes is the octet (45 us per window at 2 000 + 550 neurons; the four-lane
-    // and the earlier eight-lane form took 84 and 67 us), and HVC-RA takes
-    // octets when asked to or when the network is small enough
+    // and the earlier eight-lane form took 84 and 67 us)
     const int i_layout = nd.i_model == 0 && tu.i_lanes ? 3 : 0;
-    const int ra_lanes = tu.ra_lanes || nd.n_ra <= kRAOctMaxNeurons[nd.ra_model == 1];
-    const int ra_per_block = ra_lanes ? wpb * kRAOctNeuronsPerWave : bs;
+    const int ra_layout = ra_lanes_f64(nd.ra_model, nd.n_ra, tu.ra_lanes);
+    const int ra_per_block = ra_layout == 8 ? wpb * kRAOctNeuronsPerWave : (ra_layout == 4 ? wpb * kRANeuronsPerWave : bs);
     const int i_per_block = i_layout ? wpb * kINeuronsPerOctWave : bs;
 #endif
     int iblocks = nd.n_i == 0 ? 0 : (nd.n_i + i_per_block - 1) / i_per_block;
@@ -1444,16 +1452,20 @@ void HVC_LAUNCHER(launch_integrate)(hipStream_t st, const NetDev& nd, int t0, in
         else HVC_K(1, 0, 0);
     }
 #else
-#define HVC_KR(R)                              \
-    if (nd.i_model == 1) {                     \
-        if (ra_lanes) HVC_K(R, 1, 2);          \
-        else HVC_K(R, 1, 0);                   \
-    } else if (i_layout) {                     \
-        if (ra_lanes) HVC_K(R, 0, 10);         \
-        else HVC_K(R, 0, 8);                   \
-    } else {                                   \
-        if (ra_lanes) HVC_K(R, 0, 2);          \
-        else HVC_K(R, 0, 0);                   \
+    // (four lanes come up with RK4 only)
+#define HVC_KR(R)                                     \
+    if (nd.i_model == 1) {                            \
+        if (ra_layout == 8) HVC_K(R, 1, 2);           \
+        else if (ra_layout == 4) HVC_K(1, 1, 32);     \
+        else HVC_K(R, 1, 0);                          \
+    } else if (i_layout) {                            \
+        if (ra_layout == 8) HVC_K(R, 0, 10);          \
+        else if (ra_layout == 4) HVC_K(1, 0, 40);     \
+        else HVC_K(R, 0, 8);                          \
+    } else {                                          \
+        if (ra_layout == 8) HVC_K(R, 0, 2);           \
+        else if (ra_layout == 4) HVC_K(1, 0, 32);     \
+        else HVC_K(R, 0, 0);                          \
     }
     if (nd.ra_model == 0) {
         HVC_KR(0)

@@ -97,7 +97,7 @@ struct NoiseId {
 struct Tuning {
     int integrate_block = 64;   // threads per block of k_integrate (64, 128, 256)
     int i_lanes = 3;            // HVC-I DP8: 3 = eight lanes per neuron, 2 = four, 1 = five, 0 = one thread
-    int ra_lanes = 0;           // HVC-RA RK4: 1 = four lanes per neuron, 0 = one thread per neuron
+    int ra_lanes = 0;           // HVC-RA: 1 = several lanes per neuron, 0 = one thread (FP64: ra_lanes_f64)
     int deliver_block = 64;     // threads per block of k_deliver
     int deliver_lists = 1;      // 1: the delivery visits listed neurons only, 0: every neuron's slot table
     int sync_block = 256;       // threads per block of k_sync

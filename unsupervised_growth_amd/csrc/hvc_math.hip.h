@@ -89,6 +89,26 @@ __device__ __forceinline__ double cdiv_fast(double a, double B, DivGuard& g)
     return q;
 }
 
+// a divisor that differs between lanes: B, RN(1 / B) and the rest of 1 / B
+struct LaneDiv {
+    double B, hi, lo;
+};
+constexpr double upper_half(double x) { return 134217729.0 * x - (134217729.0 * x - x); }
+constexpr LaneDiv lane_div(double B)
+{
+    // 1 - B hi exactly, the product as p + e (Dekker 1971, Numer. Math. 18)
+    const double hi = 1.0 / B, Bh = upper_half(B), Bl = B - Bh, hh = upper_half(hi), hl = hi - hh;
+    const double p = B * hi, e = ((Bh * hh - p) + Bh * hl + Bl * hh) + Bl * hl;
+    return LaneDiv{B, hi, ((1.0 - p) - e) / B};
+}
+__device__ __forceinline__ double cdiv_lane(double a, const LaneDiv& d) { return __builtin_fma(a, d.hi, a * d.lo); }
+__device__ __forceinline__ double cdiv_lane(double a, const LaneDiv& d, DivGuard& g)
+{
+    const double q = cdiv_lane(a, d);
+    g.note(q);
+    return q;
+}
+
 // the same quotient with the IEEE fallback applied per value
 __device__ __forceinline__ double cdiv_checked(double a, double B)
 {

@@ -78,13 +78,18 @@ struct Guard : DivGuard {
 #define DIVR(a, b) ((a) / (b))
 #define EXPR(x) ::hvc::dexp(x)
 #define EXPCD(a, B) EXPR(CD(a, B))
+#define EXPCDV(a, B, invB, inv2B) EXPR(EXACT ? (a) / (B) : ::hvc::cdiv_lane((a), LaneDiv{(B), (invB), (inv2B)}, bad))
 #define HVC_FP_FAST
 #define HVC_KEEP(x)
 #define HVC_ACC(st, f, inc) st.f = st.f + inc;
 #endif
 
-// RN(log2(e) / e) of a gate's e
+// the second constant of a gate's e (EXPCDV): RN(log2(e) / e), FP64 the rest of 1 / e
+#ifdef HVC_FP32
 #define HVC_L2(e) (real)(1.4426950408889634 / (e))
+#else
+#define HVC_L2(e) ::hvc::lane_div(e).lo
+#endif
 
 // offsets c*dt of the stage times used by the steppers, in this order
 enum DecayOffset {
@@ -308,8 +313,7 @@ __device__ __forceinline__ RAK ra_rhs(Guard& bad, const RAState& s, real EL, rea
 #endif
 }
 
-// ---- HVC-RA, RK4 form, four lanes per neuron (FP32 form; FP64: hvc_oct64.hip.h) ----
-#ifdef HVC_FP32
+// ---- HVC-RA, RK4 form, four lanes per neuron ----
 // The seven gates of HH2_buffer share one form, a + c / (1 + exp(+-(v + d) / e))
 // on Vs or Vd.  Lane q of a neuron's quad evaluates gate slots 2q and 2q + 1,
 // DPP quad broadcasts hand every lane all seven, and every lane then evaluates
@@ -318,7 +322,7 @@ __device__ __forceinline__ RAK ra_rhs(Guard& bad, const RAState& s, real EL, rea
 struct RAGateSlot {
     real a, c, d, e, inv_e;   // inv_e = the form's rounding of 1 / e (as CD uses it)
     int neg, dend;            // argument -(v + d) / (v + d); v = Vd / Vs
-    real inv2_e;              // RN(log2(e) / e) (FP32 form, EXPCDV)
+    real inv2_e;              // HVC_L2
 };
 
 __constant__ RAGateSlot kRAGates[8] = {
@@ -340,7 +344,6 @@ __device__ __forceinline__ real ra_gate(Guard& bad, const RAGateSlot& g, real vs
     real q = DIVR(g.c, 1 + EXPCDV(g.neg ? -x : x, g.e, g.inv_e, g.inv2_e));
     return g.a + q;   // a = 0: 0 + q = q (q > 0)
 }
-#endif
 
 // value of lane K of the quad, in every lane of the quad (DPP quad_perm)
 template <int K>
@@ -357,12 +360,11 @@ __device__ __forceinline__ double quad_bcast(double x)
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-template <bool EXACT, bool LANES, class Slot>
+template <bool EXACT, bool LANES>
 __device__ __forceinline__ RAK ra_rhs4(Guard& bad, const RAState& s, real EL, real GCa, const RAUniform& u,
-                                       const Slot* sl, real vs, real vd, real n, real h, real r, real c,
+                                       const RAGateSlot* sl, real vs, real vd, real n, real h, real r, real c,
                                        real ca, real E)
 {
-#ifdef HVC_FP32
     if constexpr (LANES) {
         RAGates g;
         const real g0 = ra_gate<EXACT>(bad, sl[0], vs, vd);
@@ -376,13 +378,15 @@ __device__ __forceinline__ RAK ra_rhs4(Guard& bad, const RAState& s, real EL, re
         g.cI = quad_bcast<3>(g0);
         g.lI = HR(0.0);
         return ra_rhs_g<1, EXACT>(bad, s, EL, GCa, u, g, vs, vd, n, h, HR(0.0), r, c, ca, E);
-    } else
+    } else {
+#ifdef HVC_FP32
         return ra_rhs_g<1, EXACT, true>(bad, s, EL, GCa, u, ra_gates<1, EXACT, true>(bad, vs, vd), vs, vd, n, h,
                                         HR(0.0), r, c, ca, E);
 #else
-    static_assert(!LANES, "four lanes per neuron: FP32 form");
-    return ra_rhs_g<1, EXACT>(bad, s, EL, GCa, u, ra_gates<1, EXACT>(bad, vs, vd), vs, vd, n, h, HR(0.0), r, c, ca, E);
+        return ra_rhs_g<1, EXACT>(bad, s, EL, GCa, u, ra_gates<1, EXACT>(bad, vs, vd), vs, vd, n, h, HR(0.0), r, c, ca,
+                                  E);
 #endif
+    }
 }
 
 // HH2_test::Debraband_step; J* are the point-distribution values of this step
@@ -435,9 +439,9 @@ __device__ __forceinline__ void ra_debraband(Guard& bad, RAState& s, real EL, re
 }
 
 // HH2_buffer::Runge4_step (Kutta 3/8 rule); LANES: four lanes per neuron, sl = this lane's two gate slots
-template <bool EXACT, bool LANES, class Slot>
+template <bool EXACT, bool LANES>
 __device__ __forceinline__ void ra_runge4(Guard& bad, RAState& s, real EL, real GCa, const RAUniform& u,
-                                          const Slot* sl, real E_third, real E_twothird, real E_dt)
+                                          const RAGateSlot* sl, real E_third, real E_twothird, real E_dt)
 {
     HVC_FP_FAST
     const real dt = u.dt;

@@ -127,22 +127,10 @@ __device__ __forceinline__ double qconst(double a, double B)
     return EXACT ? a / B : ::hvc::cdiv2(a, B);
 }
 
-// a divisor that differs between lanes: B, RN(1 / B) and the rest of 1 / B
-struct LaneDiv {
-    double B, hi, lo;
-};
-constexpr double upper_half(double x) { return 134217729.0 * x - (134217729.0 * x - x); }
-constexpr LaneDiv lane_div(double B)
-{
-    // 1 - B hi exactly, the product as p + e (Dekker 1971, Numer. Math. 18)
-    const double hi = 1.0 / B, Bh = upper_half(B), Bl = B - Bh, hh = upper_half(hi), hl = hi - hh;
-    const double p = B * hi, e = ((Bh * hh - p) + Bh * hl + Bl * hh) + Bl * hl;
-    return LaneDiv{B, hi, ((1.0 - p) - e) / B};
-}
 template <bool EXACT>
 __device__ __forceinline__ double qlane(double a, const LaneDiv& d)
 {
-    return EXACT ? a / d.B : __builtin_fma(a, d.hi, a * d.lo);
+    return EXACT ? a / d.B : ::hvc::cdiv_lane(a, d);
 }
 
 // ---------------------------------------------------------------------------
