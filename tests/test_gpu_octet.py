@@ -90,7 +90,7 @@ def _padded(small, n_ra):
                                gca=np.concatenate([small.gca, np.linspace(0.0, 60.0, pad)]))
 
 
-@pytest.mark.parametrize("model,n_ra", [(0, 32769), (1, 16385)])
+@pytest.mark.parametrize("model,n_ra", [(0, 32769), (1, 26625)])
 def test_large_network_takes_one_thread_per_neuron(model, n_ra):
     from unsupervised_growth_amd.network import random_network
     small = random_network(5, 3, n_train=2, p_ra2i=0.5, p_i2ra=0.5, seed=4, rr=2)

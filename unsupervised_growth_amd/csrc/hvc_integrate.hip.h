@@ -1337,10 +1337,12 @@ constexpr int kIOctSharedMaxNeurons = 10240;
 // asked.  An octet's wave is short (640 instructions per Debraband step, the
 // one-thread wave 5 600 before the two-operation quotients, 4 700 with them)
 // but eight times as many are needed.  k_integrate per window beside HVC-I
-// octets (n / 3.6 of them), octets / one thread, us: Debraband 82 / 98 at
-// 20 000 neurons, 106 / 116 at 30 000, 134 / 117 at 40 000; RK4 76 / 82 at
-// 20 000, 99 / 99 at 30 000, 126 / 99 at 40 000.
-constexpr int kRAOctMaxNeurons[2] = {32768, 16384};   // by ra_model
+// octets (n / 3.6 of them), octets / one thread, us: Debraband 81 / 102 at
+// 20 000 neurons, 105 / 118 at 30 000, 119 / 120 at 34 000, 135 / 121 at
+// 40 000; RK4 76 / 79 at 20 000, 83 / 98 at 24 000, 87 / 98 at 26 000, 99 / 98
+// at 28 000, 128 / 99 at 40 000.  (The 20 000 + 5 500 RK4 growth trial in the
+// default shape: 164 ms with octets, 172 with one thread.)
+constexpr int kRAOctMaxNeurons[2] = {32768, 26624};   // by ra_model
 // HVC-RA neurons up to which "several lanes" is eight in the RK4 model, above
 // which it is four: half the waves, so two to a SIMD hold out to 21 000 neurons
 // instead of 13 000.  k_integrate per window beside HVC-I octets, four lanes /
