@@ -143,7 +143,7 @@ def test_trace_ra_sizes(model, poisson, n, steps):
     np.testing.assert_array_equal(st, ref_state)
 
 
-@pytest.mark.parametrize("n,steps", [(1, 1), (8, 32), (9, 33), (20481, 14)])
+@pytest.mark.parametrize("n,steps", [(1, 1), (8, 32), (9, 33), (24577, 14)])
 def test_trace_i_sizes(n, steps):
     from oracle_lib import i_inputs, oracle, run_i_trace
     from unsupervised_growth_amd.engine import Engine

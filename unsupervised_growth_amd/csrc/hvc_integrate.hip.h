@@ -1356,10 +1356,15 @@ int ra_lanes_f64(int ra_model, int n_ra, int ra_lanes)
     if (ra_model == 1 && ra_lanes) return n_ra <= kRAOctMaxOverQuads ? 8 : 4;
     return ra_lanes || n_ra <= kRAOctMaxNeurons[ra_model == 1] ? 8 : 1;
 }
-// HVC-I neurons up to which a trace takes octets (a trace has no launch shape):
-// beside one-thread HVC-RA waves k_integrate takes 149 us per window with
-// octets, 204 with one thread at 16 500 HVC-I neurons, 224 / 206 at 24 750
-constexpr int kIOctMaxTraces = 20480;
+// neurons up to which a trace takes octets (a trace has no launch shape and no
+// other neurons beside it), octets / one thread: hvc_trace_ra_noalloc over 64
+// steps, us: Debraband 212 / 530 at 8 000 neurons, 270 / 536 at 16 000, 537 /
+// 568 at 28 000, 559 / 572 at 32 000, 687 / 591 at 40 000; RK4 223 / 475 at
+// 8 000, 485 / 517 at 28 000, 566 / 522 at 32 000; hvc_trace_i over 40 steps, ms,
+// most of it the copies: 1.80 / 2.30 at 8 000, 6.8 / 6.9 at 24 000, 8.3 / 8.3 at
+// 28 000, 11.2 / 10.9 at 40 000.
+constexpr int kRAOctMaxTraces[2] = {32768, 28672};   // by ra_model
+constexpr int kIOctMaxTraces = 24576;
 #endif
 
 #ifdef HVC_FP32
@@ -1373,7 +1378,7 @@ void HVC_LAUNCHER(launch_trace_ra)(hipStream_t st, const NetDev& nd, int n, int 
                      uint8_t* fired)
 {
 #ifndef HVC_FP32
-    if (n <= kRAOctMaxNeurons[nd.ra_model == 1]) {
+    if (n <= kRAOctMaxTraces[nd.ra_model == 1]) {
         if (nd.ra_model == 0)
             k_trace_ra_oct<0><<<blocks_for(n, 8), 64, kTraceLds, st>>>(nd, n, n_steps, trial, EL, GCa, kick, exc_w,
                                                                        inh_g, out, fired);
