@@ -182,3 +182,27 @@ def test_fp32_one_thread_shape_on_octets(model, ra_lanes):
     for kind in ("soma", "dend", "interneuron"):
         for x, y in zip(getattr(ra, kind), getattr(rb, kind)):
             np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("model,ra_lanes", [(1, 0), (1, 1), (0, 0)])
+def test_fp32_one_thread_arithmetic_has_one_definition(model, ra_lanes):
+    """The same, state by state and bit for bit: one network alone and with idle
+    HVC-I neurons after its own, enough of them that the kernel takes one
+    thread per HVC-I neuron."""
+    from unsupervised_growth_amd.engine import Engine
+    from unsupervised_growth_amd.network import random_network
+    net = random_network(40, 37, n_train=8, p_ra2i=0.5, p_i2ra=0.3, gei_max=2.0, seed=3)
+    i = 10241
+    padded = dataclasses.replace(net, n_i=i, i2ra_ptr=np.concatenate(
+        [net.i2ra_ptr, np.full(i - net.n_i, net.i2ra_ptr[-1], np.int32)]))
+    runs = []
+    for x in (net, padded):
+        with Engine(seed=(5, 0), precision=1, trial_ms=100.0, ra_model=model) as eng:
+            eng.upload(x)
+            eng.set_tuning(i_lanes=0, ra_lanes=ra_lanes)
+            runs.append([eng.run_trial(mode=0, trial_index=k, first_trial=k == 0, mean_injection_time=10.0,
+                                       want_state=True) for k in range(2)])
+    for a, b in zip(*runs):
+        assert sum(map(len, a.interneuron)) > 0
+        np.testing.assert_array_equal(a.i_state, b.i_state[:net.n_i])
+        np.testing.assert_array_equal(a.ra_state, b.ra_state)

@@ -545,33 +545,37 @@ __device__ __forceinline__ bool rates_vd_near(real v, real& an, real& am)
     }
     return false;
 }
-template <bool EXACT>
-__device__ __forceinline__ real i_bn(real v, Guard& bad) { HVC_FP_FAST return HR(0.2) * HVC_EXPLIN(v, 25, 80); }
-template <bool EXACT>
-__device__ __forceinline__ real i_bm(real v, Guard& bad) { HVC_FP_FAST return 40 * HVC_EXPLIN(v, 47, 18); }
-// an, am, bh, ah and wInf of one neuron (one thread per neuron) from two
+// the rates of one neuron (one thread per neuron).  an, am, bh, ah and wInf from two
 // exponentials: with E = exp(-(v + 15) / 10) and F = exp(-(v + 34) / 20),
 // exp(-(v + 22) / 10) = E e^-0.7, exp(-(v + 4) / 10) = E e^1.1 and
 // exp(-v / 5) = F^4 e^6.8 (one exp2 each instead of five).  an and am as
 // quotients hold away from their zeros only: within 5 mV of v = -15 and
 // v = -22 rates_vd_near replaces them by their series.
 struct IRates {
-    real an, am, bh, ah, wInf;
+    real an, am, ah, wInf;
+    real bn, bm, bh;   // without their factors 0.2, 40 and 10 (i_gate)
 };
 __device__ __forceinline__ IRates i_rates_shared(real v)
 {
-    HVC_FP_FAST
+#pragma clang fp contract(off)
     IRates q;
     const real vn = v + HR(15.0);
     const real e = __builtin_amdgcn_exp2f(vn * (real)(-1.4426950408889634 / 10.0));
     q.an = HR(0.15) * vn * __builtin_amdgcn_rcpf(1 - e);
     q.am = (v + HR(22.0)) * __builtin_amdgcn_rcpf(__builtin_fmaf(-e, HR(0.4965853037914095), HR(1.0)));  // e^-0.7
-    q.bh = 10 * __builtin_amdgcn_rcpf(__builtin_fmaf(e, HR(3.0041660239464334), HR(1.0)));              // e^1.1
+    q.bh = __builtin_amdgcn_rcpf(__builtin_fmaf(e, HR(3.0041660239464334), HR(1.0)));                   // e^1.1
     const real f = HVC_EXPLIN(v, 34, 20);
     q.ah = HR(0.7) * f;
     const real f2 = f * f;
     q.wInf = __builtin_amdgcn_rcpf(__builtin_fmaf(f2 * f2, HR(897.8472916504176), HR(1.0)));          // e^6.8
+    q.bn = HVC_EXPLIN(v, 25, 80);
+    q.bm = HVC_EXPLIN(v, 47, 18);
     return q;
+}
+// a (1 - x) - c b x
+__device__ __forceinline__ real i_gate(real a, real c, real b, real x)
+{
+    return __builtin_fmaf(-__builtin_fmaf(c, b, a), x, a);
 }
 #undef HVC_EXPLIN
 #else
@@ -600,9 +604,9 @@ template <bool EXACT>
 __device__ __forceinline__ IK i_rhs(Guard& bad, const IState& s, real v, real n1, real m1, real h1, real w1,
                                     real e2, real e5)
 {
-    HVC_FP_FAST
-    IK k;
 #ifdef HVC_FP32
+#pragma clang fp contract(off)
+    IK k;
     // one chain of multiply-adds, as in the quad form
     const real n2 = n1 * n1;
     const real gk = __builtin_fmaf(kI_gKdr, n2 * n2, kI_gKHT * w1);
@@ -612,19 +616,18 @@ __device__ __forceinline__ IK i_rhs(Guard& bad, const IState& s, real v, real n1
     t = __builtin_fmaf(s.Ge * e2, v, t);
     t = __builtin_fmaf(s.Gi * e5, v - kI_Ei, t);
     k.V = -t;
-    auto gate = [](real a, real b, real x) { return __builtin_fmaf(-(a + b), x, a); };   // a (1 - x) - b x
     IRates q = i_rates_shared(v);
-    const real bn = i_bn<EXACT>(v, bad), bm = i_bm<EXACT>(v, bad);
-    k.h = gate(q.ah, q.bh, h1);
-    k.n = gate(q.an, bn, n1);
-    k.m = gate(q.am, bm, m1);
+    k.h = i_gate(q.ah, HR(10.0), q.bh, h1);
+    k.n = i_gate(q.an, HR(0.2), q.bn, n1);
+    k.m = i_gate(q.am, HR(40.0), q.bm, m1);
     // an and am near their zeros: the series, after the rest of the stage
     if (rates_vd_near(v, q.an, q.am)) {
-        k.n = gate(q.an, bn, n1);
-        k.m = gate(q.am, bm, m1);
+        k.n = i_gate(q.an, HR(0.2), q.bn, n1);
+        k.m = i_gate(q.am, HR(40.0), q.bm, m1);
     }
     k.w = q.wInf - w1;   // divided by tauW = 1 (exact)
 #else
+    IK k;
     real n4 = n1 * n1 * n1 * n1;
     real m3 = m1 * m1 * m1;
     k.V = -kI_gL * (v - kI_El) - kI_gNa * h1 * m3 * (v - kI_Ena) - kI_gKdr * n4 * (v - kI_Ek)
@@ -654,6 +657,155 @@ __device__ __forceinline__ IK i_rhs(Guard& bad, const IState& s, real v, real n1
 #define HVC_F6(x) CD(dt * (x), 80)
 #endif
 
+#ifdef HVC_FP32
+// One variable's stage values and final increment in the one-thread stepper's
+// arithmetic: a combination of stage derivatives is one chain of fma, written
+// out, so that its two layouts (i_dp8, i_dp8_shared) round alike whatever the
+// compiler contracts elsewhere.  Where the first two terms have opposite
+// signs, the gates round the second one's product and V the first one's.
+struct Dp8Sum {
+    real x0, dt;
+    bool isV;
+    static __device__ __forceinline__ real f(real k, real c, real sum) { return __builtin_fmaf(k, c, sum); }
+    // fma(ka, ca, kb cb), V: fma(kb, cb, ka ca)
+    __device__ __forceinline__ real pair(real ca, real ka, real cb, real kb) const
+    {
+#pragma clang fp contract(off)
+        return __builtin_fmaf(isV ? kb : ka, isV ? cb : ca, (isV ? ka : kb) * (isV ? ca : cb));
+    }
+    __device__ __forceinline__ real at(real c) const { return __builtin_fmaf(c, dt, x0); }
+#define SH_C(n, d) ((real)((double)(n) / (double)(d)))
+    __device__ __forceinline__ real s2(real k1) const { return __builtin_fmaf(k1, dt * (real)(1.0 / 18), x0); }
+    __device__ __forceinline__ real s3(real k1, real k2) const
+    {
+        return __builtin_fmaf(f(k2, HR(3.0), k1), dt * (real)(1.0 / 48), x0);
+    }
+    __device__ __forceinline__ real s4(real k1, real k3) const
+    {
+        return __builtin_fmaf(f(k3, HR(3.0), k1), dt * HR(0.03125), x0);
+    }
+    __device__ __forceinline__ real s5(real k1, real k3, real k4) const
+    {
+        return __builtin_fmaf(f(k4, HR(75.0), pair(HR(20.0), k1, -HR(75.0), k3)), dt * HR(0.015625), x0);
+    }
+    __device__ __forceinline__ real s6(real k1, real k4, real k5) const
+    {
+#pragma clang fp contract(off)
+        return __builtin_fmaf(f(k5, HR(12.0), f(k1, HR(3.0), k4 * HR(15.0))), dt * (real)(1.0 / 80), x0);
+    }
+    __device__ __forceinline__ real s7(real k1, real k4, real k5, real k6) const
+    {
+#pragma clang fp contract(off)
+        real c = f(k1, SH_C(29443841, 614563906), k4 * SH_C(77736538, 692538347));
+        c = f(k5, -SH_C(28693883, 1125000000), c);
+        return at(f(k6, SH_C(23124283, 1800000000), c));
+    }
+    __device__ __forceinline__ real s8(real k1, real k4, real k5, real k6, real k7) const
+    {
+#pragma clang fp contract(off)
+        real c = f(k1, SH_C(16016141, 946692911), k4 * SH_C(61564180, 158732637));
+        c = f(k5, SH_C(22789713, 633445777), c);
+        c = f(k6, SH_C(545815736, 2771057229), c);
+        return at(f(k7, -SH_C(180193667, 1043307555), c));
+    }
+    __device__ __forceinline__ real s9(real k1, real k4, real k5, real k6, real k7, real k8) const
+    {
+        real c = pair(SH_C(39632708, 573591083), k1, -SH_C(433636366, 683701615), k4);
+        c = f(k5, -SH_C(421739975, 2616292301), c);
+        c = f(k6, SH_C(100302831, 723423059), c);
+        c = f(k7, SH_C(790204164, 839813087), c);
+        return at(f(k8, SH_C(800635310, 3783071287), c));
+    }
+    __device__ __forceinline__ real s10(real k1, real k4, real k5, real k6, real k7, real k8, real k9) const
+    {
+        real c = pair(SH_C(246121993, 1340847787), k1, -SH_C(37695042795, 15268766246), k4);
+        c = f(k5, -SH_C(309121744, 1061227803), c);
+        c = f(k6, -SH_C(12992083, 490766935), c);
+        c = f(k7, SH_C(6005943493, 2108947869), c);
+        c = f(k8, SH_C(393006217, 1396673457), c);
+        return at(f(k9, SH_C(123872331, 1001029789), c));
+    }
+    __device__ __forceinline__ real s11(real k1, real k4, real k5, real k6, real k7, real k8, real k9, real k10) const
+    {
+        real c = pair(SH_C(8478235783, 508512852), k4, SH_C(-1028468189, 846180014), k1);
+        c = f(k5, SH_C(1311729495, 1432422823), c);
+        c = f(k6, -SH_C(10304129995, 1701304382), c);
+        c = f(k7, -SH_C(48777925059, 3047939560), c);
+        c = f(k8, SH_C(15336726248, 1032824649), c);
+        c = f(k9, -SH_C(45442868181, 3398467696), c);
+        return at(f(k10, SH_C(3065993473, 597172653), c));
+    }
+    __device__ __forceinline__ real s12(real k1, real k4, real k5, real k6, real k7, real k8, real k9, real k10,
+                                        real k11) const
+    {
+        real c = pair(SH_C(185892177, 718116043), k1, -SH_C(3185094517, 667107341), k4);
+        c = f(k5, -SH_C(477755414, 1098053517), c);
+        c = f(k6, -SH_C(703635378, 230739211), c);
+        c = f(k7, SH_C(5731566787, 1027545527), c);
+        c = f(k8, SH_C(5232866602, 850066563), c);
+        c = f(k9, -SH_C(4093664535, 808688257), c);
+        c = f(k10, SH_C(3962137247, 1805957418), c);
+        return at(f(k11, SH_C(65686358, 487910083), c));
+    }
+    // the step's end: x0 + lo plus the final combination, compensated (HVC_ACC)
+    __device__ __forceinline__ real end(real& lo, real k1, real k6, real k7, real k8, real k9, real k10, real k11,
+                                        real k12) const
+    {
+#pragma clang fp contract(off)
+        real c = pair(SH_C(13451932, 455176623), k1, -SH_C(808719846, 976000145), k6);
+        c = f(k7, SH_C(1757004468, 5645159321), c);
+        c = f(k8, SH_C(656045339, 265891186), c);
+        c = f(k9, -SH_C(3867574721, 1518517206), c);
+        c = f(k10, SH_C(465885868, 322736535), c);
+        c = f(k11, SH_C(53011238, 667516719), c);
+        c = f(k12, SH_C(2, 45), c);
+        const real y = __builtin_fmaf(c, dt, lo), x = x0 + y;
+        lo = y - (x - x0);
+        return x;
+    }
+#undef SH_C
+};
+
+// HHI_buffer::DP8_step; row = decay factors of this step
+template <bool EXACT, class Row>
+__device__ __forceinline__ void i_dp8(Guard& bad, IState& s, real dt, const Row& row)
+{
+    const IState s0 = s;
+    // the five variables' stage values: sum(member, its Dp8Sum)
+    auto all = [&](auto sum) {
+        return IK{sum(&IK::V, Dp8Sum{s0.V, dt, true}), sum(&IK::n, Dp8Sum{s0.n, dt, false}),
+                  sum(&IK::m, Dp8Sum{s0.m, dt, false}), sum(&IK::h, Dp8Sum{s0.h, dt, false}),
+                  sum(&IK::w, Dp8Sum{s0.w, dt, false})};
+    };
+    auto rhs = [&](const IK& x, int off) {
+        return i_rhs<EXACT>(bad, s, x.V, x.n, x.m, x.h, x.w, row.e2[off], row.e5[off]);
+    };
+#define HVC_ALL(call) all([&](real IK::*x, const Dp8Sum& c) { return c.call; })
+    const IK k1 = i_rhs<EXACT>(bad, s, s.V, s.n, s.m, s.h, s.w, HR(1.0), HR(1.0));
+    const IK k2 = rhs(HVC_ALL(s2(k1.*x)), kOffDp2);
+    const IK k3 = rhs(HVC_ALL(s3(k1.*x, k2.*x)), kOffDp3);
+    const IK k4 = rhs(HVC_ALL(s4(k1.*x, k3.*x)), kOffDp4);
+    const IK k5 = rhs(HVC_ALL(s5(k1.*x, k3.*x, k4.*x)), kOffDp5);
+    const IK k6 = rhs(HVC_ALL(s6(k1.*x, k4.*x, k5.*x)), kOffDp6);
+    const IK k7 = rhs(HVC_ALL(s7(k1.*x, k4.*x, k5.*x, k6.*x)), kOffDp7);
+    const IK k8 = rhs(HVC_ALL(s8(k1.*x, k4.*x, k5.*x, k6.*x, k7.*x)), kOffDp8);
+    const IK k9 = rhs(HVC_ALL(s9(k1.*x, k4.*x, k5.*x, k6.*x, k7.*x, k8.*x)), kOffDp9);
+    const IK k10 = rhs(HVC_ALL(s10(k1.*x, k4.*x, k5.*x, k6.*x, k7.*x, k8.*x, k9.*x)), kOffDp10);
+    const IK k11 = rhs(HVC_ALL(s11(k1.*x, k4.*x, k5.*x, k6.*x, k7.*x, k8.*x, k9.*x, k10.*x)), kOffDp11);
+    const IK k12 = rhs(HVC_ALL(s12(k1.*x, k4.*x, k5.*x, k6.*x, k7.*x, k8.*x, k9.*x, k10.*x, k11.*x)), kOffDt);
+#undef HVC_ALL
+    auto end = [&](real IK::*x, real x0, real& lo, bool isV) {
+        return Dp8Sum{x0, dt, isV}.end(lo, k1.*x, k6.*x, k7.*x, k8.*x, k9.*x, k10.*x, k11.*x, k12.*x);
+    };
+    s.V = end(&IK::V, s0.V, s.V_lo, true);
+    s.n = end(&IK::n, s0.n, s.n_lo, false);
+    s.m = end(&IK::m, s0.m, s.m_lo, false);
+    s.h = end(&IK::h, s0.h, s.h_lo, false);
+    s.w = end(&IK::w, s0.w, s.w_lo, false);
+    s.Ge = s.Ge * row_e2dt(row);
+    s.Gi = s.Gi * row_e5dt(row);
+}
+#else
 // HHI_buffer::DP8_step; row = decay factors of this step
 template <bool EXACT, class Row>
 __device__ __forceinline__ void i_dp8(Guard& bad, IState& s, real dt, const Row& row)
@@ -721,6 +873,7 @@ __device__ __forceinline__ void i_dp8(Guard& bad, IState& s, real dt, const Row&
 #undef C12
 #undef CF
 }
+#endif
 
 // HHI_buffer::Runge4_step
 template <bool EXACT, class Row>
@@ -1278,8 +1431,8 @@ __device__ __forceinline__ void i_dp8_oct(Guard& bad, IState& s, real& xo, real&
 // ---- the octet in the one-thread stepper's arithmetic ----
 // Where a context asks for one thread per neuron but has too few neurons to
 // fill the chip that way, the same numbers come from eight lanes: every
-// product and every fma below is the one the one-thread stepper (i_dp8) is
-// compiled to, so the bits are its bits.
+// product and every fma below is one of the one-thread stepper (Dp8Sum, i_rhs),
+// which writes out its own too, so the bits are its bits.
 //
 // The derivative of the lane's own variable but V (i_rates_shared and i_rhs):
 // with E = exp2(fma(v + d, k, k0)) of the lane,
@@ -1338,17 +1491,14 @@ struct IOctShared {
 };
 
 // HHI_buffer::DP8_step with eight lanes per neuron in i_dp8's arithmetic; as
-// i_dp8_oct.  A combination of stage derivatives is one chain of fma; where its
-// first two terms have opposite signs, i_dp8 rounds the second term's product
-// for the gates and the first's for V (whose derivative is a negated sum), so
-// V's lane takes the pair exchanged.
+// i_dp8_oct
 template <class Row>
 __device__ __forceinline__ void i_dp8_shared(IState& s, real& xo, real& xlo, int q, const IOctShared& g, real dt,
                                              const Row& row)
 {
 #pragma clang fp contract(off)
-    const real x0 = xo;
     const bool isV = q == 0;
+    const Dp8Sum c{xo, dt, isV};
     real x = xo, v = s.V, n1 = s.n, m1 = s.m, h1 = s.h, w1 = s.w;
     real e2r[11], e5r[11];
 #pragma unroll
@@ -1369,95 +1519,38 @@ __device__ __forceinline__ void i_dp8_shared(IState& s, real& xo, real& xlo, int
         const real kg = g.deriv(q, v, x);
         return isV ? -t : kg;
     };
-    auto pair = [&](real ca, real ka, real cb, real kb) {   // fma(ka, ca, kb cb), V: fma(kb, cb, ka ca)
-        return __builtin_fmaf(isV ? kb : ka, isV ? cb : ca, (isV ? ka : kb) * (isV ? ca : cb));
-    };
-#define SH_C(n, d) ((real)((double)(n) / (double)(d)))
-#define SH_F(k, c, sum) __builtin_fmaf(k, c, sum)
+#define SH_STAGE(value) \
+    x = c.value;        \
+    HVC_BCAST8(x)
     const real k1 = deriv(HR(1.0), HR(1.0));
-    x = __builtin_fmaf(k1, dt * (real)(1.0 / 18), x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s2(k1))
     const real k2 = deriv(e2r[0], e5r[0]);
-    x = __builtin_fmaf(SH_F(k2, HR(3.0), k1), dt * (real)(1.0 / 48), x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s3(k1, k2))
     const real k3 = deriv(e2r[1], e5r[1]);
-    x = __builtin_fmaf(SH_F(k3, HR(3.0), k1), dt * HR(0.03125), x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s4(k1, k3))
     const real k4 = deriv(e2r[2], e5r[2]);
-    x = __builtin_fmaf(SH_F(k4, HR(75.0), pair(HR(20.0), k1, -HR(75.0), k3)), dt * HR(0.015625), x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s5(k1, k3, k4))
     const real k5 = deriv(e2r[3], e5r[3]);
-    x = __builtin_fmaf(SH_F(k5, HR(12.0), SH_F(k1, HR(3.0), k4 * HR(15.0))), dt * (real)(1.0 / 80), x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s6(k1, k4, k5))
     const real k6 = deriv(e2r[4], e5r[4]);
-    real c = SH_F(k1, SH_C(29443841, 614563906), k4 * SH_C(77736538, 692538347));
-    c = SH_F(k5, -SH_C(28693883, 1125000000), c);
-    c = SH_F(k6, SH_C(23124283, 1800000000), c);
-    x = __builtin_fmaf(c, dt, x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s7(k1, k4, k5, k6))
     const real k7 = deriv(e2r[5], e5r[5]);
-    c = SH_F(k1, SH_C(16016141, 946692911), k4 * SH_C(61564180, 158732637));
-    c = SH_F(k5, SH_C(22789713, 633445777), c);
-    c = SH_F(k6, SH_C(545815736, 2771057229), c);
-    c = SH_F(k7, -SH_C(180193667, 1043307555), c);
-    x = __builtin_fmaf(c, dt, x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s8(k1, k4, k5, k6, k7))
     const real k8 = deriv(e2r[6], e5r[6]);
-    c = pair(SH_C(39632708, 573591083), k1, -SH_C(433636366, 683701615), k4);
-    c = SH_F(k5, -SH_C(421739975, 2616292301), c);
-    c = SH_F(k6, SH_C(100302831, 723423059), c);
-    c = SH_F(k7, SH_C(790204164, 839813087), c);
-    c = SH_F(k8, SH_C(800635310, 3783071287), c);
-    x = __builtin_fmaf(c, dt, x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s9(k1, k4, k5, k6, k7, k8))
     const real k9 = deriv(e2r[7], e5r[7]);
-    c = pair(SH_C(246121993, 1340847787), k1, -SH_C(37695042795, 15268766246), k4);
-    c = SH_F(k5, -SH_C(309121744, 1061227803), c);
-    c = SH_F(k6, -SH_C(12992083, 490766935), c);
-    c = SH_F(k7, SH_C(6005943493, 2108947869), c);
-    c = SH_F(k8, SH_C(393006217, 1396673457), c);
-    c = SH_F(k9, SH_C(123872331, 1001029789), c);
-    x = __builtin_fmaf(c, dt, x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s10(k1, k4, k5, k6, k7, k8, k9))
     const real k10 = deriv(e2r[8], e5r[8]);
-    c = pair(SH_C(8478235783, 508512852), k4, SH_C(-1028468189, 846180014), k1);
-    c = SH_F(k5, SH_C(1311729495, 1432422823), c);
-    c = SH_F(k6, -SH_C(10304129995, 1701304382), c);
-    c = SH_F(k7, -SH_C(48777925059, 3047939560), c);
-    c = SH_F(k8, SH_C(15336726248, 1032824649), c);
-    c = SH_F(k9, -SH_C(45442868181, 3398467696), c);
-    c = SH_F(k10, SH_C(3065993473, 597172653), c);
-    x = __builtin_fmaf(c, dt, x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s11(k1, k4, k5, k6, k7, k8, k9, k10))
     const real k11 = deriv(e2r[9], e5r[9]);
-    c = pair(SH_C(185892177, 718116043), k1, -SH_C(3185094517, 667107341), k4);
-    c = SH_F(k5, -SH_C(477755414, 1098053517), c);
-    c = SH_F(k6, -SH_C(703635378, 230739211), c);
-    c = SH_F(k7, SH_C(5731566787, 1027545527), c);
-    c = SH_F(k8, SH_C(5232866602, 850066563), c);
-    c = SH_F(k9, -SH_C(4093664535, 808688257), c);
-    c = SH_F(k10, SH_C(3962137247, 1805957418), c);
-    c = SH_F(k11, SH_C(65686358, 487910083), c);
-    x = __builtin_fmaf(c, dt, x0);
-    HVC_BCAST8(x)
+    SH_STAGE(s12(k1, k4, k5, k6, k7, k8, k9, k10, k11))
     const real k12 = deriv(e2r[10], e5r[10]);
-    c = pair(SH_C(13451932, 455176623), k1, -SH_C(808719846, 976000145), k6);
-    c = SH_F(k7, SH_C(1757004468, 5645159321), c);
-    c = SH_F(k8, SH_C(656045339, 265891186), c);
-    c = SH_F(k9, -SH_C(3867574721, 1518517206), c);
-    c = SH_F(k10, SH_C(465885868, 322736535), c);
-    c = SH_F(k11, SH_C(53011238, 667516719), c);
-    c = SH_F(k12, SH_C(2, 45), c);
-    const real y = __builtin_fmaf(c, dt, xlo);   // Kahan (HVC_ACC)
-    x = x0 + y;
-    xlo = y - (x - x0);
-    xo = x;
-    HVC_BCAST8(x)
+    xo = c.end(xlo, k1, k6, k7, k8, k9, k10, k11, k12);
+    HVC_BCAST8(xo)
+#undef SH_STAGE
     s.V = v; s.n = n1; s.m = m1; s.h = h1; s.w = w1;
     s.Ge = s.Ge * row_e2dt(row);
     s.Gi = s.Gi * row_e5dt(row);
-#undef SH_C
-#undef SH_F
 }
 #undef HVC_BCAST8
 #endif  // HVC_FP32
