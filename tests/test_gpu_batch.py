@@ -66,7 +66,9 @@ def test_batch_equals_each_network_alone(precision):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_launch_shapes_do_not_change_results(precision):
     """Every launch shape the autotuner may pick gives the same bits (RK4 form),
-    the delivery on its lists or sweeping every neuron."""
+    the delivery on its lists or sweeping every neuron.  (In FP64 the shapes'
+    HVC-RA layouts are one at this size, and i_lanes 1 to 3 are at any;
+    test_gpu_octet.py runs the layouts of large networks.)"""
     from unsupervised_growth_amd.engine import Engine
     nets = _nets()
     keys = [(100 + b, 7) for b in range(len(nets))]
@@ -80,7 +82,7 @@ def test_launch_shapes_do_not_change_results(precision):
               dict(integrate_block=256, i_lanes=3, deliver_block=256, sync_block=256, ra_lanes=0, deliver_lists=1)]
     runs = []
     for shape in shapes:
-        # the RK4 form for HVC-RA, where four lanes per neuron exist
+        # the RK4 form for HVC-RA, where FP32 has four lanes per neuron
         with Engine(precision=precision, trial_ms=200.0, ra_model=1) as e:
             e.upload_batch(nets, keys)
             e.set_tuning(**shape)

@@ -65,6 +65,43 @@ def test_fp32_trace_i_spikes_within_one_step():
     _check(_trains(ref_fired, 1), _trains(fi, 1), "interneuron")
 
 
+# Short traces stay near the oracle in every state variable: a step's derivatives
+# carry a few units of 2^-24 of their largest terms (hundreds of mV/ms in a
+# spike), under 2e-4 mV in V over 2 ms, and a spike's rise multiplies a deviation
+# by at most ~100: 2e-2 mV of ~100 mV.  An input of a step lost or taken twice
+# moves a conductance by 1e-2 or more.
+SHORT_TOL = 2e-4
+
+
+def _near(st, ref, what):
+    for k in range(ref.shape[2]):
+        tol = SHORT_TOL * max(1.0, float(np.abs(ref[..., k]).max()))
+        np.testing.assert_allclose(st[..., k], ref[..., k], rtol=0, atol=tol, err_msg="%s, state %d" % (what, k))
+
+
+@pytest.mark.parametrize("n,steps", [(1, 1), (7, 32), (64, 33), (65, 64), (130, 97)])
+@pytest.mark.parametrize("model,poisson", [(0, 0), (1, 1)])
+def test_fp32_trace_ra_sizes(model, poisson, n, steps):
+    """Chunk (32 steps) and block (64 neurons) edges, an input at every step."""
+    rng = np.random.default_rng(n)
+    erest, gca = ra_inputs(n, 1)[:2]
+    inp = (erest, gca, *(rng.uniform(lo, hi, (steps, n)) for lo, hi in ((0.01, 0.05), (100.0, 400.0), (0.01, 0.02))))
+    ref, _ = run_ra_trace(oracle(), "ora", model, inp, poisson=poisson, seed=(7, 0), trial=2)
+    with _engine(ra_model=model, ra_poisson=poisson, seed=(7, 0)) as eng:
+        st, _ = eng.trace_ra(*inp, trial=2)
+    _near(st, ref, "model %d" % model)
+
+
+@pytest.mark.parametrize("n,steps", [(1, 1), (7, 32), (64, 33), (65, 64), (130, 97)])
+def test_fp32_trace_i_sizes(n, steps):
+    rng = np.random.default_rng(n)
+    inp = tuple(rng.uniform(0.01, 0.03, (steps, n)) for _ in range(2))
+    ref, _ = run_i_trace(oracle(), "ora", 0, inp, first_trial=0, seed=(7, 0), trial=3)
+    with _engine(i_model=0, seed=(7, 0)) as eng:
+        st, _ = eng.trace_i(*inp, trial=3, first_trial=0)
+    _near(st, ref, "interneuron")
+
+
 def _net(seed=3, n_ra=60, n_i=16, rr="dense"):
     from unsupervised_growth_amd.network import random_network
     return random_network(n_ra, n_i, n_train=10, p_ra2i=0.3, p_i2ra=0.3, gie_max=1.0, gei_max=0.5,

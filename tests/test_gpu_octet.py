@@ -97,10 +97,10 @@ def test_large_network_takes_one_thread_per_neuron(model, n_ra):
     _compare(_padded(small, n_ra), 3.0, ra_model=model)
 
 
-@pytest.mark.parametrize("model,n_ra,ra_lanes", [(1, 14337, 1)])
+@pytest.mark.parametrize("model,n_ra,ra_lanes", [(1, 14337, 1), (0, 32769, 0), (1, 26625, 0)])
 def test_large_network_through_a_kick(model, n_ra, ra_lanes):
-    """The layouts of large networks (four lanes in the RK4 model) with their
-    spikes, deliveries and STDP: two trials kicked at their start."""
+    """The layouts of large networks (four lanes in the RK4 model, one thread)
+    with their spikes, deliveries and STDP: two trials kicked at their start."""
     from unsupervised_growth_amd.engine import Engine
     from unsupervised_growth_amd.network import random_network
     small = random_network(20, 6, n_train=8, p_ra2i=0.5, p_i2ra=0.5, seed=4, w_rr=150.0, delays=("uniform", 0.0, 2.0),

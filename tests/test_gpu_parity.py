@@ -74,9 +74,10 @@ def _compare_synapses(syn, osyn):
                                                              (12, 1, 0, 1), (12, 1, 1, 0), ("dense", 0, 0, 3),
                                                              (12, 1, 1, 3)])
 def test_growth_trials_bit_exact(rr, ra_model, ra_lanes, i_lanes):
-    """Full growth trials in every integration layout: HVC-RA (RK4 form) with
-    four lanes or one thread per neuron, HVC-I (DP8) with four, five or eight
-    lanes or one thread per neuron."""
+    """Full growth trials in the integration layouts of a small network: HVC-RA
+    with eight lanes per neuron, HVC-I (DP8) with eight lanes or one thread.
+    (The FP64 form takes eight lanes for every shape with several, and for
+    HVC-RA at this size; four lanes and one thread: test_gpu_octet.py.)"""
     net = _small_net(rr=rr)
     trial_ms = 300.0
     print("growth rr=%s ra_model=%d ra_lanes=%d i_lanes=%d n_ra=%d n_i=%d trial_ms=%g" % (
