@@ -581,11 +581,8 @@ __device__ void integrate_i_lanes(const NetDev& nd, const Win& win, int wave, in
     }
     ge = __shfl(ge, base);
     s.Ge = ge;
-    // low part of this lane's own variable (FP32 form; zero in FP64)
-    real xlo = 0;
-#ifdef HVC_FP32
-    xlo = role == 0 ? s.V_lo : (role == 1 ? s.n_lo : (role == 2 ? s.m_lo : (role == 3 ? s.h_lo : s.w_lo)));
-#endif
+    // low part of this lane's own variable
+    real xlo = role == 0 ? s.V_lo : (role == 1 ? s.n_lo : (role == 2 ? s.m_lo : (role == 3 ? s.h_lo : s.w_lo)));
     uint64_t mask = 0;
     for (int t = t0; t <= t1; ++t) {
         int f = i_state_check(s.V, flag);
@@ -603,11 +600,7 @@ __device__ void integrate_i_lanes(const NetDev& nd, const Win& win, int wave, in
     if (live) {
         // each lane writes its own variable, widened with its low part
         const real xr = role == 0 ? s.V : (role == 1 ? s.n : (role == 2 ? s.m : (role == 3 ? s.h : s.w)));
-#ifdef HVC_FP32
         nd.in[role][i] = (double)xr + (double)xlo;
-#else
-        nd.in[role][i] = xr;
-#endif
     }
     if (live && role == 0) {
         nd.in[5][i] = s.Ge; nd.in[6][i] = s.Gi;
@@ -650,12 +643,9 @@ __device__ void integrate_i_quad(const NetDev& nd, const Win& win, int wave, int
     }
     ge = quad_bcast<0>(ge);
     s.Ge = ge;
-    // low parts of this lane's variable and of w (FP32 form; zero in FP64)
-    real xlo = 0, wlo = 0;
-#ifdef HVC_FP32
-    xlo = role == 0 ? s.V_lo : (role == 1 ? s.n_lo : (role == 2 ? s.m_lo : s.h_lo));
-    wlo = s.w_lo;
-#endif
+    // low parts of this lane's variable and of w
+    real xlo = role == 0 ? s.V_lo : (role == 1 ? s.n_lo : (role == 2 ? s.m_lo : s.h_lo));
+    real wlo = s.w_lo;
     uint64_t mask = 0;
     for (int t = t0; t <= t1; ++t) {
         int f = i_state_check(s.V, flag);
@@ -673,13 +663,8 @@ __device__ void integrate_i_quad(const NetDev& nd, const Win& win, int wave, int
     if (live) {
         // each lane writes its own variable, widened with its low part; lane 0 also w
         const real xr = role == 0 ? s.V : (role == 1 ? s.n : (role == 2 ? s.m : s.h));
-#ifdef HVC_FP32
         nd.in[role][i] = (double)xr + (double)xlo;
         if (role == 0) nd.in[4][i] = (double)s.w + (double)wlo;
-#else
-        nd.in[role][i] = xr;
-        if (role == 0) nd.in[4][i] = s.w;
-#endif
     }
     if (live && role == 0) {
         nd.in[5][i] = s.Ge; nd.in[6][i] = s.Gi;

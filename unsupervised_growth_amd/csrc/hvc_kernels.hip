@@ -1100,11 +1100,11 @@ __global__ __launch_bounds__(512) void k_sync(NetDev nd)
 
 // end of a growth trial: potentiation_decay + update_all_synapses
 // (NGS:9567-9570), one wave per row.  The decay is a stream over the edges
-// (17 bytes read and 8 written each), 64 at a time; update_synapse changes
+// (10 bytes read and 8 written each), 64 at a time; update_synapse changes
 // nothing for an edge whose flags already agree with its weight, so only the
 // others take it, in the row's order, on the wave's first lane.  One thread
 // per row read a cache line per edge and array: 1 700 us at 2 000 rows of
-// 1 999 edges, now 29 us (100 MB, 3.4 TB/s); 280 -> 7 us at 300 dense rows.
+// 1 999 edges, now 29 us (72 MB, 2.5 TB/s); 280 -> 7 us at 300 dense rows.
 __global__ __launch_bounds__(256) void k_decay(NetDev nd)
 {
     const int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = __lane_id();

@@ -243,11 +243,21 @@ constexpr double kDp8D[kDp8Terms] = {
     667516719.0, 45.0};
 
 // A term is RN(RN(n k) / d): cdiv2 with its small product taken from k itself,
-// k RN(n Yl) instead of RN(n k) Yl, which moves the sum by another 2^-106 |q|
-// at most and starts it one operation earlier.  Three constants a term: what
+// k RN(n Yl) instead of RN(n k) Yl, which starts the sum one operation earlier.
+// The roundings of n Yl and of n k move the sum by another 2^-106 |q| each, four
+// such terms in all: 2^-104 |q|, under 2^-51 ulp, against ulp / (4 d_odd) to a
+// rounding boundary.  So the divisors' odd parts must stay below 2^49, and are
+// below 2^34.  Three constants a term: what
 // the compiler would otherwise build from two scalar moves each at every use
 // (227 of a step's 1 490 instructions), the first kDp8Pinned terms keep in
 // vector registers (the count that leaves two waves to a SIMD).
+constexpr bool dp8_divisors_below(double limit)
+{
+    for (double d : kDp8D)
+        if (!(d < limit)) return false;
+    return true;
+}
+static_assert(dp8_divisors_below(0x1p49), "dp8_term's error bound");
 constexpr int kDp8Pinned = 21;
 struct Dp8Consts {
     double n[kDp8Pinned], hi[kDp8Pinned], lo[kDp8Pinned];
