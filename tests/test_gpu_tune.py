@@ -68,6 +68,31 @@ def test_scratch_trials_leave_the_network(precision):
     assert sum(map(len, runs[0][0][1].soma)) > 0
 
 
+def test_pool_is_tuned_on_chain_tests():
+    """A serving pool's scratch trials are chain tests; its networks' results are
+    those of a pool that was not tuned."""
+    from unsupervised_growth_amd.configs import grown_chain_network
+    from unsupervised_growth_amd.engine import Pool, pool_caps
+    nets = [grown_chain_network(np.random.default_rng(k), 120 + 40 * k, 33 + 11 * k) for k in range(2)]
+    caps = pool_caps(max_nets=2, max_ra=400, max_i=120, max_rr=4000, max_ra2i=20000, max_i2ra=20000,
+                     max_in_degree=200, spikes_per_neuron=128)
+    runs = []
+    for tune in (False, True):
+        with Pool(caps, ra_model=1, precision=0, trial_ms=100.0) as pool:
+            handles = [pool.admit(net, (7 + k, 0)) for k, net in enumerate(nets)]
+            if tune:
+                _, ms = pool.autotune(windows=100)
+                assert (ms > 0).all()
+            trial = dict(mode=1, training=True, trial_index=0, first_trial=True, mean_injection_time=20.0)
+            res = pool.run({h: trial for h in handles})
+            runs.append([res[h] for h in handles])
+    for a, b in zip(*runs):
+        for kind in ("soma", "dend", "interneuron"):
+            for x, y in zip(getattr(a, kind), getattr(b, kind)):
+                np.testing.assert_array_equal(x, y)
+        assert sum(map(len, a.soma)) > 0
+
+
 def test_fp64_rk4_has_a_layout_between_octets_and_one_thread():
     """At 20 000 HVC-RA neurons four lanes per neuron take 61 us per window of
     k_integrate where eight take 76 and one thread 79."""
