@@ -41,10 +41,11 @@ def unpacked(achieved, precision):
 
 # HBM bytes per launch of the integration kernel, from the rocprofv3 FETCH_SIZE /
 # WRITE_SIZE passes (scaled by an elementwise kernel of known traffic) recorded in
-# profiles/integrate_c3_hbm_traffic.txt; keyed by (config, precision, HVC-I layout)
-TRAFFIC_PROFILED = {("c3", 1, 3): 7.244e6, ("c3", 0, 3): 7.680e6}
+# profiles/integrate_c3_hbm_traffic.txt; keyed by (config, precision, HVC-I layout);
+# FP64: four lanes per HVC-RA neuron, the autotuned shape
+TRAFFIC_PROFILED = {("c3", 1, 3): 7.281e6, ("c3", 0, 3): 8.589e6}
 # HBM bytes per launch of the delivery kernel (same passes), keyed by (config, delivery form: 0 sweep, 1 lists)
-DELIVER_TRAFFIC_PROFILED = {("c3", 0): 1.278e6, ("c3", 1): 1.873e6}
+DELIVER_TRAFFIC_PROFILED = {("c3", 0): 1.277e6, ("c3", 1): 1.900e6}
 DELIVER_TRAFFIC_NOTE = "profiles/integrate_c3_hbm_traffic.txt"
 HBM_PEAK_GBPS = 8000.0
 
